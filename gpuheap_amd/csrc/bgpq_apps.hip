@@ -234,6 +234,8 @@ extern "C" int bgpq_sssp(bgpq_heap* h, const int32_t* d_rowptr, const int32_t* d
     if (n_vertices < 1 || source < 0 || source >= n_vertices || !d_rowptr || !d_col || !d_w || !d_dist)
         return bgpq_fail(BGPQ_EINVAL, "sssp: bad arguments");
     hipStream_t s = (hipStream_t)stream;
+    rc = bgpq_on_stream(h, s);
+    if (rc) return rc;
     BGPQ_HIPCHK(fill_u32(d_dist, n_vertices, 0xFFFFFFFFu, s));
     (void)hipGetLastError();
     hipLaunchKernelGGL(k_app_setup, dim3(1), dim3(64), 0, s, h->app_ctl, 0ll, d_dist + source, 0u, h->ctr, 0);
@@ -256,6 +258,8 @@ extern "C" int bgpq_astar(bgpq_heap* h, const uint8_t* d_free, int32_t width, in
     if ((uint64_t)width * height * 14ull + 14ull * (width + height) >= 0xFFFFFFFFull)
         return bgpq_fail(BGPQ_EINVAL, "astar: grid too large for 32-bit costs");
     hipStream_t s = (hipStream_t)stream;
+    rc = bgpq_on_stream(h, s);
+    if (rc) return rc;
     const long long cells = (long long)width * height;
     BGPQ_HIPCHK(fill_u32(d_g, cells, 0xFFFFFFFFu, s));
     (void)hipGetLastError();
@@ -306,6 +310,8 @@ extern "C" int bgpq_knapsack(bgpq_heap* h, int32_t n, const uint32_t* weight, co
     if (pool_nodes <= 0) pool_nodes = (int64_t)std::min<uint64_t>(std::max<uint64_t>(cells, 1u << 16), 1ull << 26);
     if (pool_nodes > (int64_t)0xFFFFFFFFll) return bgpq_fail(BGPQ_EINVAL, "knapsack: pool over 2^32 nodes");
     hipStream_t s = (hipStream_t)stream;
+    rc = bgpq_on_stream(h, s);
+    if (rc) return rc;
     // one allocation: item arrays, prefix sums, dominance cells, node pool
     const size_t o_w = 0, o_v = o_w + 4 * (size_t)n, o_pw = (o_v + 4 * (size_t)n + 15) & ~(size_t)15;
     const size_t o_pv = o_pw + 8 * (size_t)(n + 1), o_cell = (o_pv + 8 * (size_t)(n + 1) + 15) & ~(size_t)15;
@@ -466,6 +472,8 @@ extern "C" int bgpq_knapsack_noalloc(bgpq_heap* h, int32_t n, const uint32_t* we
         pv[i + 1] = pv[i] + v[i];
     }
     hipStream_t s = (hipStream_t)stream;
+    rc = bgpq_on_stream(h, s);
+    if (rc) return rc;
     long long* ctl = reinterpret_cast<long long*>(base);
     const KnapNode root{0, 0, 0, 0};
     const uint32_t one = 1;

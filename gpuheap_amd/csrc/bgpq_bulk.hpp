@@ -1,0 +1,79 @@
+// Bulk insertion and bulk deletion: the calls that carry many batches.
+//
+// One insertion or deletion after the other meets every other one at the
+// root, and that chain of lock hand-offs bounds the per-batch kernels (about
+// 3 us per insertion and 4.4 us per pop at B = 1024 u32 whatever the grid,
+// 3% of HBM bandwidth).  A call with many batches does not need that order:
+// the heap after n insertions may be any valid heap over the same keys, and
+// k pops hand out the k * B smallest keys in ascending order.  So such a call
+// sorts the heap's keys (and the new ones) with a device-wide radix sort and
+// lays them out again as a heap whose slots ascend, which every variant
+// accepts: a slot's parent is always a lower slot, the partial buffer takes
+// the largest keys.
+//
+// The heap is quiescent while these kernels run (a call is ordered on its
+// stream), and every status word stays AVAIL.  No memory is allocated: the
+// sort's second buffer is the heap's own free slots, which are filled with
+// init_limits again afterwards; a heap too full for that takes the per-batch
+// path.  What the call does is decided on the device from the heap's
+// counters (BulkPlan), so nothing waits for the host.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace bgpq {
+
+constexpr int kRadix = 256;        // 8-bit digits
+constexpr int kMaxPasses = 8;      // of a u64 key
+constexpr int kBulkThreads = 512;  // of a pass's workgroup (8 waves)
+// Keys a workgroup takes at a time: 32 KB of LDS, which with the counters
+// leaves room for 3 workgroups on a CU.
+template <typename K>
+constexpr int bulk_tile() { return 32768 / (int)sizeof(K); }
+// Above this the lookback words' 30-bit counts would not do.
+constexpr long long kBulkMaxKeys = 1ll << 30;
+
+// What a bulk call does, decided by k_plan_insert / k_plan_delete.
+struct BulkPlan {
+    int go;               // 0: the per-batch kernel runs instead
+    int ascending;        // delete: the slots already ascend, no sort needed
+    int nb, pbs;          // batches and partial keys found
+    int total;            // keys sorted
+    int tiles;
+    int cut;              // delete: keys handed out, the smallest `cut`
+    int off;              // delete: where they start in the output
+    int nb_after, pbs_after;
+    int full_after;       // nb_after * B
+    long long spare;      // first key index of the free slots used
+    long long fill_lo, fill_hi;  // key range refilled with init_limits
+    int error;            // error flags to raise
+    int idle;             // a deletion found nothing (termination vote)
+    int active;           // passes that move keys
+    int order[kMaxPasses];  // position of a pass among them, -1: skipped
+    int violations, arrived;  // working words, 0 between calls
+};
+
+// Device memory of a handle's bulk calls.
+struct BulkMem {
+    BulkPlan* plan;
+    unsigned* hist;      // [kMaxPasses][kRadix] key counts, then first positions
+    unsigned* ticket;    // [kMaxPasses] next tile of a pass
+    unsigned* look[2];   // [tiles][kRadix] lookback words, alternating by pass
+    int tiles_max;
+};
+
+// One bulk call on one heap.
+template <typename K>
+struct BulkArgs {
+    K* items;
+    int* ctr;
+    K init_limits;
+    int batch_num, batch_size;
+    const K* keys;  // insert
+    long long n;
+    K* out;         // delete
+    long long out_cap, calls;
+    BulkMem mem;
+};
+
+}  // namespace bgpq

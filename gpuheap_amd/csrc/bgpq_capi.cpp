@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <climits>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -66,7 +68,32 @@ static size_t status_bytes(int batch_num) { return sizeof(int) * kWordStride * (
 static size_t ctr_bytes() { return sizeof(int) * kWordStride * CTR_WORDS; }
 
 static HeapArgs args_of(const bgpq_heap* h, long long out_cap = 0) {
-    return HeapArgs{h->items, h->status, h->ctr, h->init_limits, h->batch_num, 1, out_cap};
+    return HeapArgs{h->items, h->status, h->ctr, h->init_limits, h->batch_num, 1, out_cap, nullptr};
+}
+
+// The bulk calls' words follow the counters in one allocation.  Lookback
+// words are there for the most keys a bulk sort can take: their slots and as
+// many free ones.
+static size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
+static int bulk_tiles_max(const bgpq_heap* h) {
+    const long long tile = h->key_type == BGPQ_KEY_U64 ? bulk_tile<uint64_t>() : bulk_tile<uint32_t>();
+    const long long keys = std::min<long long>((long long)(h->batch_num + 1) * h->batch_size / 2, kBulkMaxKeys);
+    return (int)(keys / tile + 1);
+}
+static size_t bulk_fixed_bytes() {
+    return up256(ctr_bytes()) + up256(sizeof(BulkPlan)) + up256(sizeof(unsigned) * kMaxPasses * (kRadix + 1));
+}
+static size_t bulk_look_bytes(const bgpq_heap* h) { return sizeof(unsigned) * kRadix * (size_t)bulk_tiles_max(h); }
+static void set_bulk_mem(bgpq_heap* h) {
+    char* p = (char*)h->ctr + up256(ctr_bytes());
+    h->bulk.plan = (BulkPlan*)p;
+    p += up256(sizeof(BulkPlan));
+    h->bulk.hist = (unsigned*)p;
+    h->bulk.ticket = h->bulk.hist + kMaxPasses * kRadix;
+    p = (char*)h->ctr + bulk_fixed_bytes();
+    h->bulk.look[0] = (unsigned*)p;
+    h->bulk.look[1] = (unsigned*)(p + bulk_look_bytes(h));
+    h->bulk.tiles_max = bulk_tiles_max(h);
 }
 
 
@@ -76,7 +103,7 @@ static int fill_items(bgpq_heap* h, hipStream_t s) {
                                                : fill_u32(h->items, n, (uint32_t)h->init_limits, s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "fill: %s", hipGetErrorString(e));
     HIPCHK(hipMemsetAsync(h->status, 0, status_bytes(h->batch_num), s));
-    HIPCHK(hipMemsetAsync(h->ctr, 0, ctr_bytes(), s));
+    HIPCHK(hipMemsetAsync(h->ctr, 0, bulk_fixed_bytes(), s));  // and the bulk calls' working words
     return BGPQ_OK;
 }
 
@@ -84,6 +111,25 @@ static int counters(bgpq_heap* h, int* c) {
     std::vector<int> raw((size_t)kWordStride * CTR_WORDS);
     HIPCHK(hipMemcpy(raw.data(), h->ctr, ctr_bytes(), hipMemcpyDeviceToHost));
     for (int i = 0; i < CTR_WORDS; ++i) c[i] = raw[(size_t)i * kWordStride];
+    h->held = (long long)c[CTR_BATCH_COUNT] * h->batch_size + c[CTR_PARTIAL];
+    return BGPQ_OK;
+}
+
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+int bgpq_on_stream(bgpq_heap* h, hipStream_t s) {
+    if (h->used && s != h->stream) {
+        h->shared = true;
+        if (h->bulk_open && !capturing(s)) {
+            HIPCHK(hipDeviceSynchronize());
+            h->bulk_open = false;
+        }
+    }
+    h->used = true;
+    h->stream = s;
     return BGPQ_OK;
 }
 
@@ -184,7 +230,6 @@ int bgpq_create(bgpq_heap** out, int variant, int key_type, int batch_num, int b
     if (key_type == BGPQ_KEY_U32 && init_limits > 0xFFFFFFFFull)
         return fail(BGPQ_EINVAL, "init_limits does not fit u32");
     bgpq_heap* h = new bgpq_heap();
-    h->app_ctl = nullptr;
     h->variant = variant;
     h->key_type = key_type;
     h->batch_num = batch_num;
@@ -195,11 +240,12 @@ int bgpq_create(bgpq_heap** out, int variant, int key_type, int batch_num, int b
     auto alloc = [](void** p, size_t n) { return hipMalloc(p, n); };
     hipError_t e = alloc(&h->items, bytes);
     if (e == hipSuccess) e = alloc((void**)&h->status, status_bytes(batch_num));
-    if (e == hipSuccess) e = alloc((void**)&h->ctr, ctr_bytes());
+    if (e == hipSuccess) e = alloc((void**)&h->ctr, bulk_fixed_bytes() + 2 * bulk_look_bytes(h));
     if (e != hipSuccess) {
         bgpq_destroy(h);
         return fail(BGPQ_EHIP, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
     }
+    set_bulk_mem(h);
     int rc = fill_items(h, nullptr);
     if (rc == BGPQ_OK && hipStreamSynchronize(nullptr) != hipSuccess) rc = fail(BGPQ_EHIP, "sync after fill");
     if (rc != BGPQ_OK) {
@@ -221,11 +267,15 @@ void bgpq_destroy(bgpq_heap* h) {
 
 int bgpq_reset(bgpq_heap* h, void* stream) {
     if (!h) return fail(BGPQ_EINVAL, "null handle");
+    const int rc = bgpq_on_stream(h, (hipStream_t)stream);
+    if (rc) return rc;
+    h->held = 0;
     return fill_items(h, (hipStream_t)stream);
 }
 
 int bgpq_view(bgpq_heap* h, bgpq_view_t* out) {
     if (!h || !out) return fail(BGPQ_EINVAL, "null argument");
+    h->shared = true;
     out->items = h->items;
     out->status = h->status;
     out->ctr = h->ctr;
@@ -243,6 +293,8 @@ int bgpq_vote_reset(bgpq_heap* h, int busy, void* stream) {
     if (!h || busy < 0) return fail(BGPQ_EINVAL, "bad vote reset");
     const int w[2] = {busy, 0};
     hipStream_t s = (hipStream_t)stream;
+    const int rc = bgpq_on_stream(h, s);
+    if (rc) return rc;
     HIPCHK(hipMemcpyAsync(h->ctr + CTR_BUSY * kWordStride, &w[0], sizeof(int), hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(h->ctr + CTR_TERM * kWordStride, &w[1], sizeof(int), hipMemcpyHostToDevice, s));
     HIPCHK(hipStreamSynchronize(s));  // the words above are on this stack
@@ -260,6 +312,9 @@ int bgpq_terminated(bgpq_heap* h) {
 int bgpq_clear(bgpq_heap* h, void* stream) {
     if (!h) return fail(BGPQ_EINVAL, "null handle");
     hipStream_t s = (hipStream_t)stream;
+    const int rc = bgpq_on_stream(h, s);
+    if (rc) return rc;
+    h->held = 0;
     const hipError_t e =
         h->key_type == BGPQ_KEY_U64
             ? clear_u64(h->items, h->status, h->ctr, h->batch_num, h->batch_size, h->init_limits, s)
@@ -349,6 +404,62 @@ static int resolve_grid(bgpq_heap* h, int grid) { return grid > 0 ? grid : bgpq_
 
 static bool np_variant(const bgpq_heap* h) { return h->variant == BGPQ_BUITDD_NP || h->variant == BGPQ_TDITDD_NP; }
 
+// Whether `calls` insertions or pops are done together (bgpq_bulk.hpp):
+// where one after the other, at `each` us apart, would take longer than the
+// bulk kernels' launches (about 60 us) and their passes over the heap's
+// `keys` keys (u32 keys of 4 passes 16 ps each, u64 keys of 8 passes 50 ps).
+// Heap sort of 2^20 u32 keys, B = 1024: 7590 us one by one, 170 us together;
+// of 2^28, B = 8192: 367 ms and 6.6 ms; of 3 M u64 keys, B = 1024: 39.9 ms
+// and 0.41 ms.
+static bool bulk_pays(const bgpq_heap* h, long long calls, double each, long long keys) {
+    const double per_key = h->key_type == BGPQ_KEY_U64 ? 50e-6 : 16e-6;
+    return keys < kBulkMaxKeys && calls * each > 60.0 + keys * per_key;
+}
+
+// A grid of one workgroup keeps the calls' own order, one after the other;
+// keys that are not aligned to their size only the per-batch kernels take.
+static bool bulk_can(const bgpq_heap* h, const void* keys, int grid, hipStream_t s) {
+    return !h->shared && grid != 1 && s != hipStreamPerThread && (uintptr_t)keys % key_bytes(h->key_type) == 0 &&
+           !capturing(s);
+}
+
+// `sure`: the caller has seen that the plan cannot refuse.
+static int insert_calls(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, int grid, hipStream_t s, bool sure) {
+    const int rc = bgpq_on_stream(h, s);
+    if (rc) return rc;
+    HeapArgs a = args_of(h);
+    if (bulk_pays(h, (n + chunk - 1) / chunk, 2.0, h->held + n) && bulk_can(h, d_keys, grid, s)) {
+        const hipError_t e = bulk_insert(h, d_keys, n, bgpq_default_grid(h->batch_size), s);
+        if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk insert launch: %s", hipGetErrorString(e));
+        h->bulk_open = true;
+        a.skip = &h->bulk.plan->go;
+    }
+    h->held += n;
+    if (a.skip && sure) return BGPQ_OK;
+    const hipError_t e = h->row->insert(a, d_keys, n, chunk, resolve_grid(h, grid), s);
+    if (e != hipSuccess) return fail(BGPQ_EHIP, "insert launch: %s", hipGetErrorString(e));
+    return BGPQ_OK;
+}
+
+static int delete_calls(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t calls, int grid, hipStream_t s,
+                        bool sure) {
+    const int rc = bgpq_on_stream(h, s);
+    if (rc) return rc;
+    HeapArgs a = args_of(h, out_keys);
+    const long long pops = std::min<long long>(calls, (h->held + h->batch_size - 1) / h->batch_size);
+    if (bulk_pays(h, pops, 4.0, h->held) && bulk_can(h, d_out, grid, s)) {
+        const hipError_t e = bulk_delete(h, d_out, out_keys, calls, bgpq_default_grid(h->batch_size), s);
+        if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk delete launch: %s", hipGetErrorString(e));
+        h->bulk_open = true;
+        a.skip = &h->bulk.plan->go;
+    }
+    h->held = std::max<long long>(h->held - pops * h->batch_size, 0);
+    if (a.skip && sure) return BGPQ_OK;
+    const hipError_t e = h->row->del(a, d_out, calls, resolve_grid(h, grid), s);
+    if (e != hipSuccess) return fail(BGPQ_EHIP, "delete launch: %s", hipGetErrorString(e));
+    return BGPQ_OK;
+}
+
 int bgpq_insert(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, int grid, void* stream) {
     if (!h) return fail(BGPQ_EINVAL, "null handle");
     if (n < 0) return fail(BGPQ_EINVAL, "n %lld", (long long)n);
@@ -358,9 +469,7 @@ int bgpq_insert(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, int grid
     if (chunk > h->batch_size) return fail(BGPQ_EINVAL, "chunk %d > batch size %d", chunk, h->batch_size);
     if (np_variant(h) && (chunk != h->batch_size || n % h->batch_size))
         return fail(BGPQ_EINVAL, "_np variants insert full batches only (chunk %d, n %lld)", chunk, (long long)n);
-    hipError_t e = h->row->insert(args_of(h), d_keys, n, chunk, resolve_grid(h, grid), (hipStream_t)stream);
-    if (e != hipSuccess) return fail(BGPQ_EHIP, "insert launch: %s", hipGetErrorString(e));
-    return BGPQ_OK;
+    return insert_calls(h, d_keys, n, chunk, grid, (hipStream_t)stream, false);
 }
 
 int bgpq_delete(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t calls, int grid, void* stream) {
@@ -369,9 +478,7 @@ int bgpq_delete(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t calls, int 
                                                (long long)out_keys);
     if (calls == 0) return BGPQ_OK;
     if (!d_out) return fail(BGPQ_EINVAL, "null output");
-    hipError_t e = h->row->del(args_of(h, out_keys), d_out, calls, resolve_grid(h, grid), (hipStream_t)stream);
-    if (e != hipSuccess) return fail(BGPQ_EHIP, "delete launch: %s", hipGetErrorString(e));
-    return BGPQ_OK;
+    return delete_calls(h, d_out, out_keys, calls, grid, (hipStream_t)stream, false);
 }
 
 int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chunk, void* d_out, int64_t out_keys,
@@ -386,6 +493,9 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
     if (grid < 2) return fail(BGPQ_EINVAL, "concurrent run needs a grid of at least 2");
     if ((n_insert && !d_keys) || (calls && !d_out)) return fail(BGPQ_EINVAL, "null buffer");
     if (out_keys < 0) return fail(BGPQ_EINVAL, "out_keys %lld", (long long)out_keys);
+    const int rc = bgpq_on_stream(h, (hipStream_t)stream);
+    if (rc) return rc;
+    h->held = std::max<long long>(h->held + n_insert - std::min<long long>(calls, INT_MAX) * h->batch_size, 0);
     hipError_t e = h->row->conc(args_of(h, out_keys), d_keys, n_insert, chunk, d_out, calls, grid, (hipStream_t)stream);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "concurrent launch: %s", hipGetErrorString(e));
     return BGPQ_OK;
@@ -398,25 +508,35 @@ int bgpq_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n, int ch
     if (n > 0x7FFFFFFF) return fail(BGPQ_EINVAL, "the heap-sort cursor is 32-bit: n <= 2^31-1");
     hipStream_t s = (hipStream_t)stream;
     if (chunk <= 0) chunk = h->batch_size;
-    int64_t items = 0;
-    int rc = bgpq_item_count(h, &items);
+    int rc = bgpq_on_stream(h, s);
     if (rc) return rc;
+    int c[CTR_WORDS];
+    rc = counters(h, c);
+    if (rc) return rc;
+    const int64_t items = h->held;
     if (items != 0) return fail(BGPQ_EINVAL, "heap sort needs an empty heap (%lld items)", (long long)items);
     const int64_t B = h->batch_size;
     if ((n + B - 1) / B > (int64_t)h->batch_num / 2)
         return fail(BGPQ_EINVAL, "capacity: %lld keys need batch_num >= %lld", (long long)n,
                     (long long)(2 * ((n + B - 1) / B)));
+    if (chunk > h->batch_size) return fail(BGPQ_EINVAL, "chunk %d > batch size %d", chunk, h->batch_size);
+    if (np_variant(h) && n > 0 && (chunk != h->batch_size || n % h->batch_size))
+        return fail(BGPQ_EINVAL, "_np variants insert full batches only (chunk %d, n %lld)", chunk, (long long)n);
+    // the heap is empty and the keys fit twice: only an aborted heap makes
+    // a bulk call refuse
+    const bool sure = c[CTR_ABORT] == 0;
     HIPCHK(hipMemsetAsync(h->ctr + CTR_DELETE_COUNT * kWordStride, 0, sizeof(int), s));
     hipEvent_t e0, e1, e2;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipEventCreate(&e2));
     HIPCHK(hipEventRecord(e0, s));
-    rc = bgpq_insert(h, d_in, n, chunk, grid_insert, stream);
+    if (n > 0) rc = insert_calls(h, d_in, n, chunk, grid_insert, s, sure);
     if (!rc) {
         HIPCHK(hipEventRecord(e1, s));
         // enough calls to drain: every call removes a full batch or the partial buffer
-        rc = bgpq_delete(h, d_out, n, (n + B - 1) / B + 1, grid_delete, stream);
+        if (d_out) rc = delete_calls(h, d_out, n, (n + B - 1) / B + 1, grid_delete, s, sure);
+        else rc = fail(BGPQ_EINVAL, "null output");
     }
     if (!rc) {
         HIPCHK(hipEventRecord(e2, s));

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "bgpq.h"
+#include "bgpq_bulk.hpp"
 #include "bgpq_kernels.hpp"
 
 struct bgpq_heap {
@@ -18,7 +19,31 @@ struct bgpq_heap {
     int* ctr;
     const bgpq::LaunchRow* row;
     long long* app_ctl;  // driver control words, allocated on first use
+    bgpq::BulkMem bulk;  // working words of the bulk calls, behind ctr
+    // Keys the heap holds as far as the host can tell without asking the
+    // device.  It only chooses between the per-batch and the bulk kernels;
+    // those act on the counters they find.
+    long long held;
+    // The bulk kernels need the heap to themselves.  They stay off once the
+    // view was handed out (kernels of the caller may use the heap at any
+    // time) or calls came on more than one stream.
+    bool shared;
+    bool used;           // a call was made, on `stream`
+    hipStream_t stream;
+    hipEvent_t bulk_done;  // end of the last bulk call, for calls on other streams
+    bool bulk_open;
 };
+
+// To be called before work of the heap is put on a stream: notes the stream
+// and, where the stream changes, waits for a bulk call on the last one.
+int bgpq_on_stream(bgpq_heap* h, hipStream_t s);
+
+namespace bgpq {
+// The launch sequences of bgpq_bulk.hip.  A per-batch kernel with
+// HeapArgs::skip = &plan->go must follow them, unless the plan cannot refuse.
+hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, int cus, hipStream_t s);
+hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, int cus, hipStream_t s);
+}  // namespace bgpq
 
 // Records the message returned by bgpq_last_error and returns `code`.
 int bgpq_fail(int code, const char* fmt, ...);

@@ -17,7 +17,8 @@ constexpr bool batch_fits() { return delete_lds_bytes<K, B>() <= kMaxLdsBytes; }
 
 template <typename K, int VAR, int B>
 __global__ __launch_bounds__(threads_for(B)) void k_insert(HeapView<K> h, const K* keys, long long n,
-                                                           int chunk) {
+                                                           int chunk, const int* skip) {
+    if (skip && *skip) return;  // a bulk call did the work
     constexpr int NT = threads_for(B);
     DevHeap<K, VAR, B, NT> hp{h};
     const long long calls = (n + chunk - 1) / chunk;
@@ -28,7 +29,9 @@ __global__ __launch_bounds__(threads_for(B)) void k_insert(HeapView<K> h, const 
 }
 
 template <typename K, int VAR, int B>
-__global__ __launch_bounds__(threads_for(B)) void k_delete(HeapView<K> h, K* out, long long calls) {
+__global__ __launch_bounds__(threads_for(B)) void k_delete(HeapView<K> h, K* out, long long calls,
+                                                           const int* skip) {
+    if (skip && *skip) return;  // a bulk call did the work
     constexpr int NT = threads_for(B);
     DevHeap<K, VAR, B, NT> hp{h};
     for (long long i = blockIdx.x; i < calls; i += gridDim.x) {
@@ -135,6 +138,7 @@ struct HeapArgs {
     int batch_num;
     int heap_sort;
     long long out_cap;
+    const int* skip;  // insert, del: nothing to do where this word is not 0 (null: run)
 };
 
 struct LaunchRow {
@@ -171,7 +175,7 @@ struct Launch {
         if (ok != hipSuccess) return ok;
         clear_last_error();
         hipLaunchKernelGGL((k_insert<K, VAR, B>), dim3(grid), dim3(threads_for(B)), lds, s, view_of<K>(a),
-                           (const K*)keys, n, chunk);
+                           (const K*)keys, n, chunk, a.skip);
         return hipGetLastError();
     }
     static hipError_t del(const HeapArgs& a, void* out, long long calls, int grid, hipStream_t s) {
@@ -179,7 +183,7 @@ struct Launch {
         if (ok != hipSuccess) return ok;
         clear_last_error();
         hipLaunchKernelGGL((k_delete<K, VAR, B>), dim3(grid), dim3(threads_for(B)), lds, s, view_of<K>(a),
-                           (K*)out, calls);
+                           (K*)out, calls, a.skip);
         return hipGetLastError();
     }
     static hipError_t conc(const HeapArgs& a, const void* keys, long long n, int chunk, void* out,

@@ -1,0 +1,208 @@
+"""Calls that carry many batches (insertions and deletions done together by
+one radix sort, gpuheap_amd/csrc/bgpq_bulk.hpp) against the per-batch kernels
+(a grid of one workgroup never bulks) and numpy: same keys out, same
+counters, a heap the checker accepts and both kernels can go on with."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import _oracle as O
+import gpuheap_amd as G
+from gpuheap_amd import DeviceBuffer, Heap, batch_num_for
+from gpuheap_amd._lib import check, lib
+
+pytestmark = pytest.mark.gpu
+
+VARIANTS = list(G.VARIANTS)
+PB = ("buitdd", "tditdd")
+
+
+def _keys(key, n, seed, order):
+    k = O.keys_u64(seed, n) if key == "u64" else O.keys_u32(seed, n)
+    dt = k.dtype.type
+    if order == "ascending":
+        return np.sort(k)
+    if order == "descending":
+        return np.sort(k)[::-1].copy()
+    if order == "ties":
+        return (k % dt(12)) * dt(1000)
+    if order == "one":
+        return np.full(n, 77, k.dtype)
+    if order == "byte2":  # one digit differs: every other pass is skipped
+        return ((k % dt(256)) << dt(16)) + dt(3)
+    return k
+
+
+def _held(snapshot, B):
+    """The keys of a heap in ascending order."""
+    items, _, ctr = snapshot
+    return np.sort(np.concatenate([items[:ctr[1]], items[B:B * (ctr[0] + 1)]]))
+
+
+def _valid(h, keys):
+    """The heap holds exactly these keys, in order for its checker."""
+    assert h.checkInsertHeap(), h.last_check_message
+    items, status, ctr = h.snapshot()
+    B = h.batch_size
+    assert not status.any() and ctr[3] == 0
+    assert (ctr[0], ctr[1]) == (len(keys) // B, len(keys) % B)
+    assert np.array_equal(_held((items, status, ctr), B), np.sort(keys))
+    free = np.concatenate([items[ctr[1]:B], items[B * (ctr[0] + 1):]])
+    assert (free == h.dtype.type(h.init_limits)).all(), "a free slot does not hold init_limits"
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("key,B", [("u32", 64), ("u32", 1024), ("u32", 8192), ("u64", 128), ("u64", 4096)])
+@pytest.mark.parametrize("order", ["random", "ascending", "descending", "ties", "one", "byte2"])
+def test_bulk_sort_orders(gpu, variant, key, B, order):
+    # tiles of the passes hold 8192 u32 or 4096 u64 keys: counts around whole
+    # tiles, the last tile one key, nearly full, full
+    tile = 8192 if key == "u32" else 4096
+    for n in (40 * tile, 40 * tile + 1, 43 * tile - 1):
+        if variant not in PB:
+            n = -(-n // B) * B
+        n = max(n, 150 * B)
+        print(f"[case] bulk {variant} {key} B={B} {order} n={n}", flush=True)
+        keys = _keys(key, n, 5, order)
+        h = Heap(batch_num_for(n, B), B, variant=variant, key=key)
+        d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer(keys.nbytes)
+        h.insert(d, n)
+        _valid(h, keys)
+        h.delete(out, n // B + 1)
+        G.sync()
+        assert h.isEmpty() and h.error_flags() == 0
+        assert np.array_equal(out.to_numpy(keys.dtype, n), np.sort(keys))
+        _valid(h, keys[:0])
+        h.close()
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("key", ["u32", "u64"])
+def test_bulk_and_per_batch_calls_mixed(gpu, variant, key):
+    """Bulk and per-batch calls on one heap in turn: bulk insertions into a
+    heap the per-batch kernel filled and the reverse, partial drains of both
+    kinds from ascending and from walked heaps; each pop equals the same
+    calls on a heap driven by one workgroup."""
+    B = 128
+    pb = variant in PB
+    rng = np.random.default_rng(3)
+    a = Heap(4096, B, variant=variant, key=key)
+    b = Heap(4096, B, variant=variant, key=key)
+    cap = 1 << 20
+    outs = [DeviceBuffer(cap * a.dtype.itemsize) for _ in range(2)]
+    held = 0
+    for step, (what, calls) in enumerate([("i", 3), ("i", 400), ("d", 2), ("d", 300), ("i", 5), ("i", 200), ("d", 150),
+                                          ("d", 4), ("i", 900), ("d", 1), ("d", 700), ("i", 150), ("d", 5000)]):
+        print(f"[case] bulk mixed {variant} {key} step {step} {what}{calls}", flush=True)
+        if what == "i":
+            chunk = int(rng.integers(B // 2, B + 1)) if pb else B
+            n = calls * chunk - (int(rng.integers(1, chunk)) if pb else 0)
+            keys = _keys(key, n, 100 + step, "ties" if step == 5 else "random")
+            d = DeviceBuffer.from_numpy(keys)
+            a.insert(d, n, chunk=chunk)
+            b.insert(d, n, chunk=chunk, grid=1)
+        else:
+            a.delete(outs[0], calls)
+            b.delete(outs[1], calls, grid=1)
+        G.sync()
+        assert a.checkInsertHeap(), a.last_check_message
+        sa, sb = a.snapshot(), b.snapshot()
+        assert np.array_equal(sa[2][:4], sb[2][:4])
+        assert np.array_equal(_held(sa, B), _held(sb, B))
+        done = sa[2][2]
+        assert np.array_equal(outs[0].to_numpy(a.dtype, done), outs[1].to_numpy(a.dtype, done))
+        # a few pops by one workgroup from the bulk heap's layout
+        if what == "i":
+            a.delete(outs[0], 2, grid=1)
+            b.delete(outs[1], 2, grid=1)
+            G.sync()
+            assert a.checkInsertHeap(), a.last_check_message
+    assert a.isEmpty() and b.isEmpty()
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+def test_bulk_limits(gpu, variant):
+    """What a bulk call must leave to the per-batch kernels or report like
+    them: a heap without room for the sort's second buffer, one without room
+    for the keys, an output that ends early, an init_limits below the type's
+    largest, pointers not aligned to 16 bytes."""
+    B, calls = 64, 600
+    n = B * calls
+    keys = O.keys_u32(21, n) >> np.uint32(1)
+    d = DeviceBuffer.from_numpy(keys)
+    print(f"[case] bulk limits {variant}: full heap", flush=True)
+    h = Heap(calls, B, variant=variant, init_limits=1 << 31)
+    h.insert(d, n)
+    _valid(h, keys)
+    h.insert(d, 300 * B)  # no slot left: overflow, nothing lost
+    G.sync()
+    assert h.error_flags() & 1 and h.nodeCount() == calls
+    h.reset()
+    h.insert(d, n)
+    _valid(h, keys)
+    out = DeviceBuffer(n * 4)
+    h.delete(out, calls + 3)
+    G.sync()
+    assert h.isEmpty() and np.array_equal(out.to_numpy(np.uint32, n), np.sort(keys))
+    print(f"[case] bulk limits {variant}: short output, odd alignment", flush=True)
+    for spare in (0, 1):  # without and with room for a sort
+        h = Heap(calls * (2 if spare else 1) + 2, B, variant=variant, init_limits=1 << 31)
+        h.insert(d, n - B, grid=0)
+        h.insert(d.ptr + 4 * (n - B), B, grid=1)
+        h.set_cursor(3)
+        room = 500 * B + 7
+        out = DeviceBuffer(4 * n)
+        mark = np.full(n, 0xABCDABCD, np.uint32)
+        out.upload(mark)
+        h.delete(out.ptr + 4, calls, out_keys=room)
+        G.sync()
+        assert h.error_flags() & 16
+        got = out.to_numpy(np.uint32, n)
+        m = (room - 3) // B * B
+        assert np.array_equal(got[4:4 + m], np.sort(keys)[:m])
+        assert (got[:4] == mark[0]).all() and (got[4 + m:] == mark[0]).all()
+        assert h.itemCount() == n - m
+        h.close()
+
+
+def test_bulk_needs_the_heap_to_itself(gpu):
+    """After its view was handed out a heap takes the per-batch kernels only:
+    the words of a walked heap differ from the ascending layout."""
+    B, n = 64, 64 * 1000
+    keys = O.keys_u32(4, n)
+    d = DeviceBuffer.from_numpy(keys)
+
+    def ascends(h):
+        items = h.snapshot()[0][B:B * (n // B + 1)]
+        return bool((items[1:] >= items[:-1]).all())
+
+    h = Heap(4096, B)
+    h.insert(d, n)
+    assert ascends(h)
+    g = Heap(4096, B)
+    g.view()
+    g.insert(d, n)
+    assert not ascends(g) and g.checkInsertHeap()
+    out = DeviceBuffer(n * 4)
+    g.delete(out, n // B)
+    G.sync()
+    assert np.array_equal(out.to_numpy(np.uint32, n), np.sort(keys))
+
+
+def test_bulk_calls_on_two_streams(gpu):
+    """A call on another stream follows a bulk call on the first."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    s = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+    B, n = 1024, 1 << 22
+    keys = O.keys_u32(6, n)
+    d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer(n * 4)
+    h = Heap(batch_num_for(n, B), B)
+    h.insert(d, n)
+    check(lib().bgpq_delete(h._h, out.ptr, n, n // B + 1, 0, s))
+    assert hip.hipStreamSynchronize(s) == 0
+    assert np.array_equal(out.to_numpy(np.uint32, n), np.sort(keys))
+    assert h.isEmpty()
+    h.close()
+    assert hip.hipStreamDestroy(s) == 0
