@@ -16,17 +16,17 @@ namespace bgpq {
 template <int VAR, int B>
 __global__ __launch_bounds__(threads_for(B)) void k_sssp(HeapView<uint64_t> h, SsspApp app, long long* ctl,
                                                          uint64_t first) {
-    drive<VAR, B, threads_for(B)>(h, app, ctl, first, blockIdx.x == 0);
+    drive<VAR, B, threads_for(B)>(h, app, ctl, first, blockIdx.x == 0, (int)gridDim.x);
 }
 template <int VAR, int B>
 __global__ __launch_bounds__(threads_for(B)) void k_astar(HeapView<uint64_t> h, AstarApp app, long long* ctl,
                                                           uint64_t first) {
-    drive<VAR, B, threads_for(B)>(h, app, ctl, first, blockIdx.x == 0);
+    drive<VAR, B, threads_for(B)>(h, app, ctl, first, blockIdx.x == 0, (int)gridDim.x);
 }
 template <int VAR, int B>
 __global__ __launch_bounds__(threads_for(B)) void k_knapsack(HeapView<uint64_t> h, KnapsackApp app,
                                                              long long* ctl, uint64_t first) {
-    drive<VAR, B, threads_for(B)>(h, app, ctl, first, blockIdx.x == 0);
+    drive<VAR, B, threads_for(B)>(h, app, ctl, first, blockIdx.x == 0, (int)gridDim.x);
 }
 
 // Control words to their start state, plus one 32-bit label set (the

@@ -126,25 +126,25 @@ __device__ __forceinline__ int sys_load(const int* p) {
 }
 
 // One solve, inlined into its tier's kernel: as calls (noinline) the
-// solves took 216-246 VGPRs at 512 threads, inlined the kernel takes 162,
+// solves took 216-246 VGPRs at 512 threads, inlined the kernel takes 168,
 // so both tiers' workgroups fit on a CU together.
 template <int B, int NT>
 __device__ __forceinline__ void solve_sssp(const QueryDesc& d, bool first) {
     const HeapView<uint64_t> hv{d.items, d.status, d.ctr, ~0ull, (int)d.batch_num, 0, 0};
     const SsspApp app{d.rowptr, d.col, d.w, d.labels, d.ctl};
-    drive<VAR_BUITDD, B, NT>(hv, app, d.ctl, d.first_key, first);
+    drive<VAR_BUITDD, B, NT>(hv, app, d.ctl, d.first_key, first, d.team);
 }
 template <int B, int NT>
 __device__ __forceinline__ void solve_astar(const QueryDesc& d, bool first) {
     const HeapView<uint64_t> hv{d.items, d.status, d.ctr, ~0ull, (int)d.batch_num, 0, 0};
     const AstarApp app{d.free_cells, d.n, d.height, d.labels, d.ctl};
-    drive<VAR_BUITDD, B, NT>(hv, app, d.ctl, d.first_key, first);
+    drive<VAR_BUITDD, B, NT>(hv, app, d.ctl, d.first_key, first, d.team);
 }
 template <int B, int NT>
 __device__ __forceinline__ void solve_knapsack(const QueryDesc& d, bool first) {
     const HeapView<uint64_t> hv{d.items, d.status, d.ctr, ~0ull, (int)d.batch_num, 0, 0};
     const KnapsackApp app{d.n, d.cap, d.kw, d.kv, d.pw, d.pv, d.cell, d.pool, d.pool_cap, d.ctl};
-    drive<VAR_BUITDD, B, NT>(hv, app, d.ctl, d.first_key, first);
+    drive<VAR_BUITDD, B, NT>(hv, app, d.ctl, d.first_key, first, d.team);
 }
 template <int B, int NT>
 __device__ __forceinline__ void solve_b(const QueryDesc& d, bool first) {
@@ -329,8 +329,10 @@ __device__ void finish(const QueryDesc& d, Completion* c) {
 // `mirror` to what it saw: reads of pinned host memory by every idle
 // workgroup of the chip (hundreds, each every few microseconds) slowed the
 // workgroups that were solving about fivefold.
+// At least 3 waves on a SIMD: 168 registers, so that a workgroup of each tier
+// fits on a CU (8 and 4 waves over 4 SIMDs of 512 registers).
 template <int NT>
-__global__ __launch_bounds__(NT) void k_serve(ServeRing r) {
+__global__ __launch_bounds__(NT, 3) void k_serve(ServeRing r) {
     __shared__ long long s_slot;
     __shared__ int s_go, s_last;
     __shared__ uint32_t s_entry;

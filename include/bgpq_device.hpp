@@ -171,6 +171,14 @@ struct DevHeap {
     // Lane 0: this workgroup's vote, busy since its last pop (counted in
     // CTR_BUSY) until a deleteRoot finds nothing to hand out.
     mutable int busy_ = 0;
+    // Lane 0: set by a workgroup that holds keys of the search outside the
+    // heap: a deleteRoot that finds nothing is then no idle vote.
+    mutable int hold_ = 0;
+    // Set by exchangeRoot for the sift that follows: lanes 0, 1: the locks of
+    // the root's children requested ahead; all: both children are in LDS.
+    mutable int pre_root_ = INT_MIN;  // kNoPre
+    mutable int pre_word_[2] = {0, 0};
+    mutable bool pre_ready_ = false;
     // Lane 0: the ticket this workgroup holds status[0] with.
     mutable unsigned t0_ = 0;
 
@@ -421,6 +429,7 @@ struct DevHeap {
             }
             return;
         }
+        if (hold_) return;
         int now = a_load(ctr(CTR_BUSY));
         if (busy_) {
             busy_ = 0;
@@ -591,15 +600,17 @@ struct DevHeap {
         K* X0 = lds_ws(smemOffset);  // candidate carried down the tree
         K* X1 = X0 + B;              // smaller half of the children
         K* X2 = X1 + B;
-        int* bc = bcast_slots();
         if (!op_begin()) return;
-        if (pre_last_ > 0) {
-            // deleteRoot already took the candidate and released status[0]
-            pre_last_ = 0;
-            sift_down(X0, X1, X2);
-            return;
-        }
+        // deleteRoot may have taken the candidate and released status[0]
+        if (pre_last_ > 0) pre_last_ = 0;
+        else if (!take_candidate(X0, X1)) return;
+        sift_down(X0, X1, X2);
+    }
 
+    // The last batch, with the smaller keys of the partial buffer, as the
+    // candidate X0; releases status[0].  False when nothing is left to sift.
+    __device__ __forceinline__ bool take_candidate(K* X0, K* X1) const {
+        int* bc = bcast_slots();
         if (threadIdx.x == 0) {
             const int last = a_add(ctr(CTR_BATCH_COUNT), -1);
             if (last == 1) {
@@ -611,13 +622,13 @@ struct DevHeap {
         __syncthreads();
         const int last = bc[BC_A];
         __syncthreads();
-        if (last == 1) return;
+        if (last == 1) return false;
 
         // ---- take the last batch as the candidate
         if constexpr (BU) {
             if (threadIdx.x == 0) lock_max(last);
             __syncthreads();
-            if (aborted()) return;
+            if (aborted()) return false;
             take_batch<K, B, NT>(X0, node(last), h.init_limits);
             publish();
             if (threadIdx.x == 0) release_st(last, AVAIL);
@@ -638,7 +649,7 @@ struct DevHeap {
                 bc[BC_B] = type;
             }
             __syncthreads();
-            if (aborted()) return;
+            if (aborted()) return false;
             const int type = bc[BC_B];
             if (type == 1) {
                 g2l_batch<K, B, NT>(X0, node(1));
@@ -666,7 +677,118 @@ struct DevHeap {
         if constexpr (PB && kSplitFold) {
             if (fold) fold_small(X0, X1);
         }
-        sift_down(X0, X1, X2);
+        return true;
+    }
+
+    // The partial buffer's keys (fewer than B) move to dst (LDS); returns how
+    // many.  A workgroup that exchanges does this first: as long as the
+    // partial buffer holds keys, every exchange has to fold it under
+    // status[0] and the root's lock.
+    __device__ int takePartial(K* dst) const {
+        int* bc = bcast_slots();
+        if (!PB || !op_begin()) return 0;
+        if (threadIdx.x == 0) {
+            bc[BC_A] = lock0() ? a_load(ctr(CTR_PARTIAL)) : 0;
+            bc[BC_B] = aborted();
+        }
+        __syncthreads();
+        const int pbs = bc[BC_A];
+        const bool gone = bc[BC_B] != 0;
+        __syncthreads();
+        if (gone) return 0;
+        for (int i = threadIdx.x; i < pbs; i += NT) {
+            dst[i] = gload_key(node(0) + i);
+            gstore_key(node(0) + i, h.init_limits);
+        }
+        publish();
+        if (threadIdx.x == 0) {
+            if (pbs > 0) a_store(ctr(CTR_PARTIAL), 0);
+            unlock0();
+        }
+        return pbs;
+    }
+
+    // ------------------------------------------------------------ exchangeRoot
+    // An insertion and a deletion in one descent: the `size` smallest keys of
+    // the root's batch and the `size` keys of `items` (1..B of them, in LDS,
+    // any order) come back ascending in out[B - size .. B) (LDS, B keys), the
+    // root keeps the B largest, and deleteUpdate(smemOffset) must follow,
+    // which sifts them down.  The heap keeps its size and no other batch
+    // moves, where an insertion walks up from a new slot and a deletion takes
+    // the last batch down again.  Returns false, with nothing changed, when
+    // the heap holds no full batch.
+    __device__ bool exchangeRoot(const K* items, int size, K* out, int smemOffset) const {
+        K* X0 = lds_ws(smemOffset);
+        K* X1 = X0 + B;
+        int* bc = bcast_slots();
+        pre_last_ = 0;
+        if (!op_begin()) return false;
+        // padded with the smallest key: the padding leaves with the smaller half
+        wg_sort_batch<K, B, NT>(X0, items, size, K(0));
+        if (threadIdx.x == 0) {
+            int mode = 0;
+            if (lock0()) {
+                // one round trip for the counters and the first attempt at the root
+                const int nb = a_load(ctr(CTR_BATCH_COUNT));
+                const int pbs = PB ? a_load(ctr(CTR_PARTIAL)) : 0;
+                const bool got = a_cas(st(1), AVAIL, INUSE);
+                if (nb == 0) {
+                    if (got) release_st(1, AVAIL);
+                    unlock0();
+                } else if (got || lock_cas_eager(1, AVAIL, INUSE)) {
+                    if (pbs == 0) unlock0();
+                    mode = pbs == 0 ? 1 : 2;
+                }
+            }
+            bc[BC_A] = mode;
+        }
+        __syncthreads();
+        const int mode = bc[BC_A];
+        if (aborted() || mode == 0) {
+            __syncthreads();
+            return false;
+        }
+        // The root is held from here until the sift's first step has stored
+        // its new batch, and every other pop waits for it: the children's
+        // locks are requested with the root's load, and their batches load
+        // during the merge.
+        int pre = kNoPre;
+        if constexpr (BU) pre = lock_ahead(1);
+        BatchLoad<K, B, NT> rl;
+        rl.issue(node(1));
+        if (BU && threadIdx.x < 2) bc[BC_C + threadIdx.x] = pre;
+        rl.commit(out);
+        __syncthreads();
+        const int lp = BU ? bc[BC_C] : kNoPre, rp = BU ? bc[BC_D] : kNoPre;
+        const bool fetch = held_ahead(lp) && held_ahead(rp);
+        BatchLoad<K, B, NT> fl, fr;
+        if (fetch) {
+            fl.issue(node(left_child(1)));
+            fr.issue(node(right_child(1)));
+        }
+        wg_merge<K, B, NT>(X0, out, ToLds<K>{out}, ToLds<K>{X0});
+        if constexpr (PB) {
+            // the partial buffer stays above the root: it takes the largest
+            if (mode == 2) {
+                g2l_batch<K, B, NT>(X1, node(0));
+                __syncthreads();
+                wg_merge<K, B, NT>(X0, X1, ToLds<K>{X0}, ToGlobal<K>{node(0)});
+                publish();
+                if (threadIdx.x == 0) unlock0();
+            }
+        }
+        if (fetch) {
+            fl.commit(X1);
+            fr.commit(X1 + B);
+            __syncthreads();
+            pre = kNoPre;
+            pre_word_[0] = is_inshold(lp) ? DELMOD : lp;
+            pre_word_[1] = is_inshold(rp) ? DELMOD : rp;
+        }
+        pre_ready_ = fetch;
+        pre_root_ = pre;
+        pre_last_ = 1;  // the candidate is in LDS, status[0] released
+        return true;
     }
 
     // Smallest batch size whose level steps take the two merge halves one
@@ -824,9 +946,11 @@ struct DevHeap {
         int cur = 1;
         int cur_prev = AVAIL;
         int pend = 0, pend_word = AVAIL;  // stored, released with the next publish
-        int pre = kNoPre;                 // lanes 0, 1: result of lock_ahead
-        bool ready = false;               // X1, X2 hold cur's children, already locked
-        int ready_lp = AVAIL, ready_rp = AVAIL;
+        int pre = pre_root_;              // lanes 0, 1: result of lock_ahead
+        bool ready = pre_ready_;          // X1, X2 hold cur's children, already locked
+        int ready_lp = pre_word_[0], ready_rp = pre_word_[1];
+        pre_root_ = kNoPre;
+        pre_ready_ = false;
         while (true) {
             const int l = left_child(cur), r = right_child(cur);
             const bool lin = l <= h.batch_num, rin = r <= h.batch_num;

@@ -1,0 +1,49 @@
+"""The drivers' loop where workgroups hold children and exchange them with the
+root's batch: team sizes from one workgroup (which may never insert) to more
+workgroups than batches, batch sizes with and without the split sift, both
+partial-buffer variants; results equal the CPU oracles' and the heap is left
+empty and valid."""
+import numpy as np
+import pytest
+
+import _oracle as O
+from gpuheap_amd import apps as A
+from gpuheap_amd import Heap
+
+pytestmark = pytest.mark.gpu
+
+
+def _heap(B, keys, variant):
+    bn = 1
+    while bn * B < 2 * keys + 128 * B:
+        bn <<= 1
+    return Heap(bn, B, variant=variant, key="u64")
+
+
+@pytest.mark.parametrize("variant", ["buitdd", "tditdd"])
+@pytest.mark.parametrize("B", [256, 512, 1024, 2048])
+@pytest.mark.parametrize("grid", [1, 2, 7, 96])
+def test_teams(gpu, variant, B, grid):
+    print(f"[case] exchange {variant} B={B} grid={grid}: sssp", flush=True)
+    rowptr, col, w = A.rmat_csr(13, 16, B + grid)
+    with _heap(B, len(col), variant) as h:
+        dist, st = A.sssp(h, A.Graph(rowptr, col, w), source=0, grid=grid)
+        assert np.array_equal(dist, O.dijkstra(rowptr, col, w, 0))
+        assert st["popped"] == st["expanded"] + st["stale"] == st["pushed"]
+        assert h.isEmpty() and h.checkInsertHeap(), h.last_check_message
+    print(f"[case] exchange {variant} B={B} grid={grid}: astar", flush=True)
+    free = A.grid_map(311, 187, 0.25, B + grid)
+    with _heap(B, 8 * 311 * 187, variant) as h:
+        gm = A.GridMap(free, 311, 187)
+        want, _ = O.astar(free, 311, 187)
+        for _ in range(2):  # the second solve starts from the cleared heap
+            cost, st = A.astar(h, gm, grid=grid)
+            assert cost == want
+            assert st["popped"] <= st["pushed"] and h.isEmpty()
+    print(f"[case] exchange {variant} B={B} grid={grid}: knapsack", flush=True)
+    w, v, cap = A.knapsack_instance(60, B + grid)
+    with _heap(B, 1 << 18, variant) as h:
+        best, st = A.knapsack(h, w, v, cap, grid=grid)
+        assert best == O.knapsack_dp(w, v, cap)
+        assert st["popped"] == st["expanded"] + st["stale"] + st["pruned"] == st["pushed"]
+        assert h.isEmpty()
