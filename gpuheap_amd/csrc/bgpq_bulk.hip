@@ -85,34 +85,66 @@ __device__ __forceinline__ bool last_to_arrive(int* arrived) {
     return s_last != 0;
 }
 
+// The plan's part that a call's pops decide: a.calls of them from nb batches
+// and pbs partial keys, whole batches first and the partial buffer only once
+// no batch is left, as many as the output holds.  The slots in use end below
+// `spare`; `through` keys pass through the free slots from there on.
+template <typename K>
+__device__ __forceinline__ void plan_pops(const BulkArgs<K>& a, BulkPlan& pl, long long nb, int pbs, long long spare,
+                                          bool ascending) {
+    const long long B = a.batch_size, total = nb * B + pbs, off = ctr_of(a, CTR_DELETE_COUNT);
+    long long pops = a.calls < nb ? a.calls : nb;
+    const long long room = off <= a.out_cap ? (a.out_cap - off) / B : 0;
+    int error = 0;
+    if (pops > room) {
+        pops = room;
+        error = ERR_OUTPUT_FULL;
+    }
+    bool last = pops == nb && a.calls > nb && pbs > 0;
+    if (last && off + total > a.out_cap) {
+        last = false;
+        error = ERR_OUTPUT_FULL;
+    }
+    const long long cut = pops * B + (last ? pbs : 0);
+    const long long tiles = (total + bulk_tile<K>() - 1) / bulk_tile<K>();
+    pl.total = (int)total;
+    pl.tiles = (int)tiles;
+    pl.ascending = ascending;
+    pl.cut = (int)cut;
+    pl.off = (int)off;
+    pl.nb_after = (int)(nb - pops);
+    pl.pbs_after = last ? 0 : pbs;
+    pl.full_after = (int)((nb - pops) * B);
+    // a sort moves every key through the free slots, ascending slots only
+    // the batches that stay (the partial buffer stays where it is)
+    const long long through = ascending ? (nb - pops) * B : total;
+    pl.spare = spare;
+    pl.fill_lo = (nb - pops + 1) * B;
+    pl.fill_hi = spare + through;
+    pl.error = error;
+    pl.idle = a.calls > pops + (last ? 1 : 0) && total == cut;
+    pl.go = total > 0 && total < kBulkMaxKeys && tiles <= a.mem.tiles_max &&
+            spare + through <= ((long long)a.batch_num + 1) * B && (cut == 0 || off + total < (1ll << 31)) &&
+            ctr_of(a, CTR_ABORT) == 0;
+}
+
+// Insertions, and pops after them where the call has any (a concurrent call,
+// whose insertions and pops may take effect in any order).
 template <typename K>
 __global__ __launch_bounds__(256) void k_plan_insert(BulkArgs<K> a) {
     BulkPlan& pl = *a.mem.plan;
     clear_sort_words(a.mem);
     if (threadIdx.x != 0) return;
     const int B = a.batch_size, nb = ctr_of(a, CTR_BATCH_COUNT), pbs = ctr_of(a, CTR_PARTIAL);
-    const long long total = (long long)nb * B + pbs + a.n;
-    const long long full = total / B;
+    const long long total = (long long)nb * B + pbs + a.n, full = total / B;
     pl.nb = nb;
     pl.pbs = pbs;
-    pl.total = (int)total;
-    const long long tiles = (total + bulk_tile<K>() - 1) / bulk_tile<K>();
-    pl.tiles = (int)tiles;
-    // every key fits, and the free slots past them hold the second buffer
-    pl.go = total < kBulkMaxKeys && tiles <= a.mem.tiles_max && full <= a.batch_num &&
-            (a.batch_num - full) * B >= total && ctr_of(a, CTR_ABORT) == 0;
-    pl.ascending = 0;
-    pl.cut = pl.off = 0;
-    pl.nb_after = (int)full;
-    pl.pbs_after = (int)(total % B);
-    pl.full_after = (int)(full * B);
-    pl.spare = pl.fill_lo = (full + 1) * B;
-    pl.fill_hi = pl.spare + total;
-    pl.error = pl.idle = 0;
+    plan_pops(a, pl, full, (int)(total % B), (full + 1) * B, false);
+    if (full > a.batch_num) pl.go = 0;
 }
 
-// Besides the plan: do the slots ascend already (a bulk insertion leaves
-// them so)?  Each batch ascends by itself, so only the borders are compared.
+// Pops alone.  Do the slots ascend already (a bulk insertion leaves them so)?
+// Each batch ascends by itself, so only the borders are compared.
 template <typename K>
 __global__ __launch_bounds__(256) void k_plan_delete(BulkArgs<K> a) {
     BulkPlan& pl = *a.mem.plan;
@@ -127,47 +159,13 @@ __global__ __launch_bounds__(256) void k_plan_delete(BulkArgs<K> a) {
     if (!last_to_arrive(&pl.arrived)) return;
     clear_sort_words(a.mem);
     if (threadIdx.x != 0) return;
-    const bool asc = a_load(&pl.violations) == 0;
+    const bool ascending = a_load(&pl.violations) == 0;
     a_store(&pl.violations, 0);
     a_store(&pl.arrived, 0);
-    const long long off = ctr_of(a, CTR_DELETE_COUNT), total = (long long)nb * B + pbs;
-    // whole batches first; the partial buffer only once no batch is left
-    long long pops = a.calls < nb ? a.calls : nb;
-    const long long room = off <= a.out_cap ? (a.out_cap - off) / B : 0;
-    int error = 0;
-    if (pops > room) {
-        pops = room;
-        error = ERR_OUTPUT_FULL;
-    }
-    bool last = pops == nb && a.calls > nb && pbs > 0;
-    if (last && off + total > a.out_cap) {
-        last = false;
-        error = ERR_OUTPUT_FULL;
-    }
-    const long long cut = pops * B + (last ? pbs : 0);
-    const long long left = total - cut;
     pl.nb = nb;
     pl.pbs = pbs;
-    pl.total = (int)total;
-    const long long tiles = (total + bulk_tile<K>() - 1) / bulk_tile<K>();
-    pl.tiles = (int)tiles;
-    pl.ascending = asc;
-    pl.cut = (int)cut;
-    pl.off = (int)off;
-    pl.nb_after = (int)(nb - pops);
-    pl.pbs_after = last ? 0 : pbs;
-    pl.full_after = pl.nb_after * B;
-    // a sort moves every key through the free slots, ascending slots only
-    // the batches that stay (the partial buffer stays where it is)
-    const long long through = asc ? (long long)pl.full_after : total;
-    pl.spare = (long long)(nb + 1) * B;
-    pl.fill_lo = (long long)(pl.nb_after + 1) * B;
-    pl.fill_hi = pl.spare + (cut ? through : 0);
-    pl.error = error;
-    pl.idle = a.calls > pops + (last ? 1 : 0) && left == 0;
-    pl.go = cut > 0 && total < kBulkMaxKeys && tiles <= a.mem.tiles_max &&
-            (long long)(a.batch_num - nb) * B >= through && off + total < (1ll << 31) &&
-            ctr_of(a, CTR_ABORT) == 0;
+    plan_pops(a, pl, nb, pbs, (nb + 1ll) * B, ascending);
+    if (pl.cut == 0) pl.go = 0;  // nothing to do but what the per-batch kernel reports
 }
 
 // Key counts of each digit.  A wave whose keys agree on a digit (ordered or
@@ -486,10 +484,14 @@ BulkArgs<K> args_for(const bgpq_heap* h) {
 }
 
 template <typename K>
-hipError_t insert_as(const bgpq_heap* h, const void* keys, long long n, int cus, hipStream_t s) {
+hipError_t insert_as(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap, long long calls,
+                     int cus, hipStream_t s) {
     BulkArgs<K> a = args_for<K>(h);
     a.keys = (const K*)keys;
     a.n = n;
+    a.out = (K*)out;
+    a.out_cap = out_cap;
+    a.calls = calls;
     clear_last_error();
     hipLaunchKernelGGL(k_plan_insert<K>, dim3(1), dim3(256), 0, s, a);
     return sort_and_finish(a, h->held + n, cus, s);
@@ -508,9 +510,10 @@ hipError_t delete_as(const bgpq_heap* h, void* out, long long out_cap, long long
 
 }  // namespace
 
-hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, int cus, hipStream_t s) {
-    return h->key_type == BGPQ_KEY_U64 ? insert_as<uint64_t>(h, keys, n, cus, s)
-                                       : insert_as<uint32_t>(h, keys, n, cus, s);
+hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap,
+                       long long calls, int cus, hipStream_t s) {
+    return h->key_type == BGPQ_KEY_U64 ? insert_as<uint64_t>(h, keys, n, out, out_cap, calls, cus, s)
+                                       : insert_as<uint32_t>(h, keys, n, out, out_cap, calls, cus, s);
 }
 hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, int cus, hipStream_t s) {
     return h->key_type == BGPQ_KEY_U64 ? delete_as<uint64_t>(h, out, out_cap, calls, cus, s)

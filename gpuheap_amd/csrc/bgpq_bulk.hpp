@@ -40,8 +40,8 @@ struct BulkPlan {
     int nb, pbs;          // batches and partial keys found
     int total;            // keys sorted
     int tiles;
-    int cut;              // delete: keys handed out, the smallest `cut`
-    int off;              // delete: where they start in the output
+    int cut;              // keys handed out, the smallest `cut`
+    int off;              // where they start in the output
     int nb_after, pbs_after;
     int full_after;       // nb_after * B
     long long spare;      // first key index of the free slots used
@@ -69,9 +69,9 @@ struct BulkArgs {
     int* ctr;
     K init_limits;
     int batch_num, batch_size;
-    const K* keys;  // insert
+    const K* keys;  // inserted
     long long n;
-    K* out;         // delete
+    K* out;         // popped, by `calls` deletions
     long long out_cap, calls;
     BulkMem mem;
 };

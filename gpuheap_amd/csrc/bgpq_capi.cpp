@@ -71,9 +71,12 @@ static HeapArgs args_of(const bgpq_heap* h, long long out_cap = 0) {
     return HeapArgs{h->items, h->status, h->ctr, h->init_limits, h->batch_num, 1, out_cap, nullptr};
 }
 
-// The bulk calls' words follow the counters in one allocation.  Lookback
-// words are there for the most keys a bulk sort can take: their slots and as
-// many free ones.
+// The bulk calls' words follow the counters and, for their lookback, the
+// slots, in the same allocations.  Lookback words are there for the most keys
+// a bulk sort can take: their slots and as many free ones.
+static size_t items_bytes(const bgpq_heap* h) {
+    return key_bytes(h->key_type) * (size_t)h->batch_size * (size_t)(h->batch_num + 1);
+}
 static size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 static int bulk_tiles_max(const bgpq_heap* h) {
     const long long tile = h->key_type == BGPQ_KEY_U64 ? bulk_tile<uint64_t>() : bulk_tile<uint32_t>();
@@ -90,7 +93,7 @@ static void set_bulk_mem(bgpq_heap* h) {
     p += up256(sizeof(BulkPlan));
     h->bulk.hist = (unsigned*)p;
     h->bulk.ticket = h->bulk.hist + kMaxPasses * kRadix;
-    p = (char*)h->ctr + bulk_fixed_bytes();
+    p = (char*)h->items + up256(items_bytes(h));
     h->bulk.look[0] = (unsigned*)p;
     h->bulk.look[1] = (unsigned*)(p + bulk_look_bytes(h));
     h->bulk.tiles_max = bulk_tiles_max(h);
@@ -236,11 +239,11 @@ int bgpq_create(bgpq_heap** out, int variant, int key_type, int batch_num, int b
     h->batch_size = batch_size;
     h->init_limits = init_limits;
     h->row = &rows_for(key_type, variant)[bi];
-    const size_t bytes = key_bytes(key_type) * (size_t)batch_size * (size_t)(batch_num + 1);
+    const size_t bytes = up256(items_bytes(h)) + 2 * bulk_look_bytes(h);
     auto alloc = [](void** p, size_t n) { return hipMalloc(p, n); };
     hipError_t e = alloc(&h->items, bytes);
     if (e == hipSuccess) e = alloc((void**)&h->status, status_bytes(batch_num));
-    if (e == hipSuccess) e = alloc((void**)&h->ctr, bulk_fixed_bytes() + 2 * bulk_look_bytes(h));
+    if (e == hipSuccess) e = alloc((void**)&h->ctr, bulk_fixed_bytes());
     if (e != hipSuccess) {
         bgpq_destroy(h);
         return fail(BGPQ_EHIP, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
@@ -429,7 +432,7 @@ static int insert_calls(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, 
     if (rc) return rc;
     HeapArgs a = args_of(h);
     if (bulk_pays(h, (n + chunk - 1) / chunk, 2.0, h->held + n) && bulk_can(h, d_keys, grid, s)) {
-        const hipError_t e = bulk_insert(h, d_keys, n, bgpq_default_grid(h->batch_size), s);
+        const hipError_t e = bulk_insert(h, d_keys, n, nullptr, 0, 0, bgpq_default_grid(h->batch_size), s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk insert launch: %s", hipGetErrorString(e));
         h->bulk_open = true;
         a.skip = &h->bulk.plan->go;
@@ -493,10 +496,23 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
     if (grid < 2) return fail(BGPQ_EINVAL, "concurrent run needs a grid of at least 2");
     if ((n_insert && !d_keys) || (calls && !d_out)) return fail(BGPQ_EINVAL, "null buffer");
     if (out_keys < 0) return fail(BGPQ_EINVAL, "out_keys %lld", (long long)out_keys);
-    const int rc = bgpq_on_stream(h, (hipStream_t)stream);
+    hipStream_t s = (hipStream_t)stream;
+    const int rc = bgpq_on_stream(h, s);
     if (rc) return rc;
-    h->held = std::max<long long>(h->held + n_insert - std::min<long long>(calls, INT_MAX) * h->batch_size, 0);
-    hipError_t e = h->row->conc(args_of(h, out_keys), d_keys, n_insert, chunk, d_out, calls, grid, (hipStream_t)stream);
+    HeapArgs a = args_of(h, out_keys);
+    // together: the insertions first, then the pops, one of the orders that
+    // the concurrent kernel may take
+    const long long in = (n_insert + chunk - 1) / chunk, all = h->held + n_insert;
+    const long long pops = std::min<long long>(calls, (all + h->batch_size - 1) / h->batch_size);
+    if (bulk_pays(h, in + pops, 3.0, all) && bulk_can(h, d_keys, grid, s) && bulk_can(h, d_out, grid, s)) {
+        const hipError_t e =
+            bulk_insert(h, d_keys, n_insert, d_out, out_keys, calls, bgpq_default_grid(h->batch_size), s);
+        if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk launch: %s", hipGetErrorString(e));
+        h->bulk_open = true;
+        a.skip = &h->bulk.plan->go;
+    }
+    h->held = std::max<long long>(all - pops * h->batch_size, 0);
+    hipError_t e = h->row->conc(a, d_keys, n_insert, chunk, d_out, calls, grid, s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "concurrent launch: %s", hipGetErrorString(e));
     return BGPQ_OK;
 }

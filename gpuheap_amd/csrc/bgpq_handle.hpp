@@ -19,7 +19,7 @@ struct bgpq_heap {
     int* ctr;
     const bgpq::LaunchRow* row;
     long long* app_ctl;  // driver control words, allocated on first use
-    bgpq::BulkMem bulk;  // working words of the bulk calls, behind ctr
+    bgpq::BulkMem bulk;  // working words of the bulk calls, behind ctr and items
     // Keys the heap holds as far as the host can tell without asking the
     // device.  It only chooses between the per-batch and the bulk kernels;
     // those act on the counters they find.
@@ -41,7 +41,9 @@ int bgpq_on_stream(bgpq_heap* h, hipStream_t s);
 namespace bgpq {
 // The launch sequences of bgpq_bulk.hip.  A per-batch kernel with
 // HeapArgs::skip = &plan->go must follow them, unless the plan cannot refuse.
-hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, int cus, hipStream_t s);
+// bulk_insert: n keys in, then `calls` deletions (0 for none).
+hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap,
+                       long long calls, int cus, hipStream_t s);
 hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, int cus, hipStream_t s);
 }  // namespace bgpq
 

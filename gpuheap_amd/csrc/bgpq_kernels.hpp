@@ -42,7 +42,9 @@ __global__ __launch_bounds__(threads_for(B)) void k_delete(HeapView<K> h, K* out
 
 template <typename K, int VAR, int B>
 __global__ __launch_bounds__(threads_for(B)) void k_concurrent(HeapView<K> h, const K* keys, long long n,
-                                                               int chunk, K* out, long long calls) {
+                                                               int chunk, K* out, long long calls,
+                                                               const int* skip) {
+    if (skip && *skip) return;  // a bulk call did the work
     constexpr int NT = threads_for(B);
     DevHeap<K, VAR, B, NT> hp{h};
     const int half = (int)gridDim.x / 2;
@@ -138,7 +140,7 @@ struct HeapArgs {
     int batch_num;
     int heap_sort;
     long long out_cap;
-    const int* skip;  // insert, del: nothing to do where this word is not 0 (null: run)
+    const int* skip;  // nothing to do where this word is not 0 (null: run)
 };
 
 struct LaunchRow {
@@ -192,7 +194,7 @@ struct Launch {
         if (ok != hipSuccess) return ok;
         clear_last_error();
         hipLaunchKernelGGL((k_concurrent<K, VAR, B>), dim3(grid), dim3(threads_for(B)), lds, s,
-                           view_of<K>(a), (const K*)keys, n, chunk, (K*)out, calls);
+                           view_of<K>(a), (const K*)keys, n, chunk, (K*)out, calls, a.skip);
         return hipGetLastError();
     }
     static hipError_t sort(const void* in, const int* sizes, void* out, uint64_t pad, int batches, hipStream_t s) {

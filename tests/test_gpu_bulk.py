@@ -122,6 +122,41 @@ def test_bulk_and_per_batch_calls_mixed(gpu, variant, key):
 
 
 @pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("key", ["u32", "u64"])
+@pytest.mark.parametrize("held,new,pops,room", [(0, 300, 200, 400), (200, 150, 350, 400), (200, 150, 500, 400),
+                                                (250, 200, 300, 260), (300, 0, 290, 400), (120, 300, 0, 1)])
+def test_bulk_concurrent(gpu, variant, key, held, new, pops, room):
+    """A concurrent call: ascending pops, nothing lost, a valid heap left."""
+    print(f"[case] bulk concurrent {variant} {key} held={held} new={new} pops={pops} room={room}", flush=True)
+    B = 256
+    part = 91 if variant in PB else 0  # a partial buffer, and another of 82 keys more
+    n0, n1 = held * B + (part if held else 0), new * B + (part if new else 0)
+    chunk = B // 2 if variant in PB else B
+    keys = _keys(key, n0 + n1, held + pops, "random")
+    h = Heap(1024, B, variant=variant, key=key)
+    d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer((room * B + 5) * keys.itemsize)
+    if n0:
+        h.insert(d, n0)
+    h.concurrent(d.ptr + n0 * keys.itemsize, n1, out, pops, chunk=chunk)
+    G.sync()
+    snap = h.snapshot()
+    done = int(snap[2][2])
+    batches, rest = divmod(n0 + n1, B)
+    want = min(pops, batches, room) * B
+    if pops > batches and room >= batches:
+        want += rest
+    assert done == want
+    assert bool(snap[2][3] & 16) == (min(pops, batches) > room)
+    got = out.to_numpy(keys.dtype, done)
+    assert (got[1:] >= got[:-1]).all()
+    left = _held(snap, B)
+    assert np.array_equal(np.sort(np.concatenate([got, left])), np.sort(keys))
+    if not snap[2][3]:
+        assert h.checkInsertHeap(), h.last_check_message
+    h.close()
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
 def test_bulk_limits(gpu, variant):
     """What a bulk call must leave to the per-batch kernels or report like
     them: a heap without room for the sort's second buffer, one without room
