@@ -287,22 +287,15 @@ __device__ void drive(HeapView<uint64_t> h, const App& app, long long* ctl, uint
         }
         if (hp.aborted()) break;
         if (n > 0 && size == 0) {
+            // the first m children were exchanged, or are popped themselves;
+            // the rest moves up by m = B places, up to 2B of them where the
+            // partial buffer's keys came in
             m = n < B ? n : B;
-            K rest[P];
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const int i = p * NT + t;
-                if (m + i < n) rest[p] = emit[m + i];
-                if (!sift && i < m) popped[i] = emit[i];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const int i = p * NT + t;
-                if (m + i < n) emit[i] = rest[p];
-            }
+            if (!sift)
+                for (int i = t; i < m; i += NT) popped[i] = emit[i];
             size = m;
             n -= m;
+            for (int i = t; i < n; i += NT) emit[i] = emit[B + i];  // a thread reads each place before it writes it
             if (t == 0) s_n = n;
         }
         if (sift) hp.deleteUpdate(kWs);
