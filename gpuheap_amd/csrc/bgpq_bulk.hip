@@ -1,15 +1,22 @@
 // Kernels of the bulk insertion and deletion (bgpq_bulk.hpp) and their
 // launch sequences.
 //
-//   k_plan_insert | k_plan_delete   what to do (BulkPlan), counters cleared
+// A sort (insertions, pops from slots in heap order):
+//   k_plan_delete                   pops only: what to do (BulkPlan)
 //   k_bulk_hist                     key counts of every digit of every pass
+//                                   (and the plan, where there are insertions)
 //   k_bulk_pass, once per digit     one pass of a least-digit-first radix sort
 //   k_bulk_finish                   free slots refilled, counters set
+// or, for insertions that make no more than a tile of keys in all, with pops or
+// without, k_bulk_tile alone.
+// Pops from slots that ascend, as a bulk call leaves them:
+//   k_plan_delete, k_bulk_copy, k_bulk_finish
 //
 // The passes follow the published single-pass scheme (decoupled look-back:
 // Merrill and Garland, 2016; a radix pass on it: Adinets and Merrill, 2022):
 // one read and one write of the keys per pass, where separate count and
 // scatter kernels would read them twice.
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include "bgpq_device.hpp"
@@ -68,12 +75,6 @@ __device__ __forceinline__ K* final_place(const BulkArgs<K>& a, const BulkPlan& 
     return j < pl.full_after ? a.items + a.batch_size + j : a.items + (j - pl.full_after);
 }
 
-// Counters of the sort back to zero (one workgroup).
-__device__ __forceinline__ void clear_sort_words(const BulkMem& m) {
-    for (int i = threadIdx.x; i < kMaxPasses * kRadix; i += blockDim.x) m.hist[i] = 0;
-    if (threadIdx.x < kMaxPasses) m.ticket[threadIdx.x] = 0;
-}
-
 // The workgroup that arrives last at a grid-wide counter: it sees what the
 // others added before they arrived (device-scope atomics and loads only).
 __device__ __forceinline__ bool last_to_arrive(int* arrived) {
@@ -92,7 +93,7 @@ __device__ __forceinline__ bool last_to_arrive(int* arrived) {
 template <typename K>
 __device__ __forceinline__ void plan_pops(const BulkArgs<K>& a, BulkPlan& pl, long long nb, int pbs, long long spare,
                                           bool ascending) {
-    const long long B = a.batch_size, total = nb * B + pbs, off = ctr_of(a, CTR_DELETE_COUNT);
+    const long long B = a.batch_size, total = nb * B + pbs, off = a.from_empty ? 0 : ctr_of(a, CTR_DELETE_COUNT);
     long long pops = a.calls < nb ? a.calls : nb;
     const long long room = off <= a.out_cap ? (a.out_cap - off) / B : 0;
     int error = 0;
@@ -110,6 +111,7 @@ __device__ __forceinline__ void plan_pops(const BulkArgs<K>& a, BulkPlan& pl, lo
     pl.total = (int)total;
     pl.tiles = (int)tiles;
     pl.ascending = ascending;
+    pl.drains = total == cut;
     pl.cut = (int)cut;
     pl.off = (int)off;
     pl.nb_after = (int)(nb - pops);
@@ -129,18 +131,15 @@ __device__ __forceinline__ void plan_pops(const BulkArgs<K>& a, BulkPlan& pl, lo
 }
 
 // Insertions, and pops after them where the call has any (a concurrent call,
-// whose insertions and pops may take effect in any order).
+// whose insertions and pops may take effect in any order, or a heap sort).
 template <typename K>
-__global__ __launch_bounds__(256) void k_plan_insert(BulkArgs<K> a) {
-    BulkPlan& pl = *a.mem.plan;
-    clear_sort_words(a.mem);
-    if (threadIdx.x != 0) return;
+__device__ __forceinline__ void plan_insert(const BulkArgs<K>& a, BulkPlan& pl) {
     const int B = a.batch_size, nb = ctr_of(a, CTR_BATCH_COUNT), pbs = ctr_of(a, CTR_PARTIAL);
     const long long total = (long long)nb * B + pbs + a.n, full = total / B;
     pl.nb = nb;
     pl.pbs = pbs;
     plan_pops(a, pl, full, (int)(total % B), (full + 1) * B, false);
-    if (full > a.batch_num) pl.go = 0;
+    if (full > a.batch_num || (a.from_empty && (nb | pbs) != 0)) pl.go = 0;
 }
 
 // Pops alone.  Do the slots ascend already (a bulk insertion leaves them so)?
@@ -155,35 +154,44 @@ __global__ __launch_bounds__(256) void k_plan_delete(BulkArgs<K> a) {
         if (i + 1 < nb) bad |= a.items[(i + 2) * B] < end;
         else if (pbs > 0) bad |= a.items[0] < end;
     }
-    if (__any(bad) && __lane_id() == 0) a_add(&pl.violations, 1);
-    if (!last_to_arrive(&pl.arrived)) return;
-    clear_sort_words(a.mem);
+    if (__any(bad) && __lane_id() == 0) a_add(a.mem.sync, 1);
+    if (!last_to_arrive(a.mem.sync + 1)) return;
     if (threadIdx.x != 0) return;
-    const bool ascending = a_load(&pl.violations) == 0;
-    a_store(&pl.violations, 0);
-    a_store(&pl.arrived, 0);
+    const bool ascending = a_load(a.mem.sync) == 0;
+    a_store(a.mem.sync, 0);
+    a_store(a.mem.sync + 1, 0);
     pl.nb = nb;
     pl.pbs = pbs;
     plan_pops(a, pl, nb, pbs, (nb + 1ll) * B, ascending);
-    if (pl.cut == 0) pl.go = 0;  // nothing to do but what the per-batch kernel reports
+    // nothing to do but what the per-batch kernel reports, or a sort that was not launched
+    if (pl.cut == 0 || !(ascending || a.sorts)) pl.go = 0;
 }
 
-// Key counts of each digit.  A wave whose keys agree on a digit (ordered or
-// small keys: the high digits) adds its 64 at once instead of serialising on
-// one word.  The last workgroup turns the counts into first positions and
-// drops the passes whose digit is the same for all keys; the number of
-// passes left is made even, so that the sort ends where it began.
+// Key counts of each digit: LDS atomics, of which a wave whose keys agree on
+// a digit (ordered or small keys: the high digits) makes one instead of 64 on
+// one word.  The rows of 64 keys are looked at one by one only where the first
+// agrees; a test of every row cost as much as the atomics.  The last
+// workgroup turns the counts into first positions and drops the passes whose
+// digit is the same for all keys.  The first pass must not write where keys
+// are read, so at least two are left; an even number, so that the sort ends
+// where it began, unless the last pass hands every key out.
 template <typename K>
 __global__ __launch_bounds__(256) void k_bulk_hist(BulkArgs<K> a) {
     constexpr int P = (int)sizeof(K), U = 16;
     __shared__ unsigned h[P][kRadix];
     __shared__ unsigned part[4];
     __shared__ int moves[P];
-    BulkPlan& pl = *a.mem.plan;
-    if (!pl.go || pl.ascending) return;
-    const int t = threadIdx.x, total = pl.total;
+    __shared__ BulkPlan pl;
+    const int t = threadIdx.x;
+    if (t == 0) {
+        if (a.planned) pl = *a.mem.plan;
+        else plan_insert(a, pl);
+        if (!pl.go && blockIdx.x == 0) a.mem.plan->go = 0;
+    }
     for (int i = t; i < P * kRadix; i += 256) (&h[0][0])[i] = 0;
     __syncthreads();
+    if (!pl.go || pl.ascending) return;
+    const int total = pl.total;
     // the first pass's lookback words
     for (long long i = blockIdx.x * 256ll + t; i < (long long)pl.tiles * kRadix; i += gridDim.x * 256ll)
         a.mem.look[0][i] = 0;
@@ -193,23 +201,25 @@ __global__ __launch_bounds__(256) void k_bulk_hist(BulkArgs<K> a) {
         if (const K* src = source_run(a, pl, (int)j0, 256 * U)) {
 #pragma unroll
             for (int u = 0; u < U; ++u) k[u] = src[j + u * 256];
-        } else {
-#pragma unroll
-            for (int u = 0; u < U; ++u) k[u] = j + u * 256 < total ? *source_key(a, pl, j + u * 256) : K(0);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const bool in = j + u * 256 < total;
-            const bool whole = __ballot(in) == ~0ull;
 #pragma unroll
             for (int p = 0; p < P; ++p) {
-                const int d = digit_of(k[u], p);
-                const int d0 = __builtin_amdgcn_readfirstlane(d);
-                if (whole && __ballot(d == d0) == ~0ull) {
-                    if (__lane_id() == 0) atomicAdd(&h[p][d0], 64u);
-                } else if (in) {
-                    atomicAdd(&h[p][d], 1u);
+                if (__ballot(digit_of(k[0], p) == __builtin_amdgcn_readfirstlane(digit_of(k[0], p))) != ~0ull) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) atomicAdd(&h[p][digit_of(k[u], p)], 1u);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int d = digit_of(k[u], p), d0 = __builtin_amdgcn_readfirstlane(d);
+                        if (__ballot(d == d0) != ~0ull) atomicAdd(&h[p][d], 1u);
+                        else if (__lane_id() == 0) atomicAdd(&h[p][d0], 64u);
+                    }
                 }
+            }
+        } else {
+            for (int u = 0; u < U && j + u * 256 < total; ++u) {
+                const K key = *source_key(a, pl, j + u * 256);
+#pragma unroll
+                for (int p = 0; p < P; ++p) atomicAdd(&h[p][digit_of(key, p)], 1u);
             }
         }
     }
@@ -218,11 +228,14 @@ __global__ __launch_bounds__(256) void k_bulk_hist(BulkArgs<K> a) {
         const unsigned c = (&h[0][0])[i];
         if (c) __hip_atomic_fetch_add(a.mem.hist + i, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (!last_to_arrive(&pl.arrived)) return;
+    if (!last_to_arrive(a.mem.sync + 1)) return;
     const int lane = t & 63, w = t >> 6;
+    unsigned c[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) c[p] = look_load(a.mem.hist + p * kRadix + t);
+#pragma unroll
     for (int p = 0; p < P; ++p) {
-        const unsigned c = look_load(a.mem.hist + p * kRadix + t);
-        unsigned x = c;
+        unsigned x = c[p];
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             const unsigned y = __shfl_up(x, o, 64);
@@ -231,16 +244,16 @@ __global__ __launch_bounds__(256) void k_bulk_hist(BulkArgs<K> a) {
         if (lane == 63) part[w] = x;
         if (t == 0) moves[p] = 1;
         __syncthreads();
-        if (c == (unsigned)total) moves[p] = 0;
+        if (c[p] == (unsigned)total) moves[p] = 0;
         unsigned before = 0;
         for (int i = 0; i < w; ++i) before += part[i];
-        a.mem.hist[p * kRadix + t] = x - c + before;
+        a.mem.hist[p * kRadix + t] = x - c[p] + before;
         __syncthreads();
     }
     if (t == 0) {
         int n = 0;
         for (int p = 0; p < P; ++p) n += moves[p];
-        for (int p = 0; p < P && (n < 2 || (n & 1)); ++p) {
+        for (int p = 0; p < P && (n < 2 || ((n & 1) && !pl.drains)); ++p) {
             if (!moves[p]) {
                 moves[p] = 1;
                 ++n;
@@ -249,15 +262,22 @@ __global__ __launch_bounds__(256) void k_bulk_hist(BulkArgs<K> a) {
         int at = 0;
         for (int p = 0; p < P; ++p) pl.order[p] = moves[p] ? at++ : -1;
         pl.active = n;
-        a_store(&pl.arrived, 0);
+        // where all keys leave, the output is the second buffer, so that the
+        // slots in use need no refill twice as long as the keys
+        pl.through_out = pl.drains && (n & 1) == 0;
+        if (pl.through_out && pl.nb == 0 && pl.pbs == 0) pl.fill_lo = pl.spare;
+        *a.mem.plan = pl;
+        a_store(a.mem.sync + 1, 0);
     }
 }
 
 // The slots already ascend: keys to be handed out go to the output, batches
 // that stay to the spare slots (k_bulk_finish brings them back).
 template <typename K>
-__device__ void copy_ascending(const BulkArgs<K>& a, const BulkPlan& pl) {
+__global__ __launch_bounds__(kBulkThreads) void k_bulk_copy(BulkArgs<K> a) {
     constexpr int U = 8;
+    const BulkPlan& pl = *a.mem.plan;
+    if (!pl.go || !pl.ascending) return;
     const int full = pl.nb * a.batch_size, moved = pl.cut + pl.full_after;
     const long long step = (long long)gridDim.x * kBulkThreads * U;
     for (long long j0 = (long long)blockIdx.x * (kBulkThreads * U); j0 < moved; j0 += step) {
@@ -276,6 +296,64 @@ __device__ void copy_ascending(const BulkArgs<K>& a, const BulkPlan& pl) {
     }
 }
 
+// Ranks of the wave's keys, U rows of 64, among those of the same digit, in
+// order, and the digits' counts in `mine` (zeroed before).  About 80 vector
+// instructions and 3 LDS accesses a row.  A lane finds the lanes with its
+// digit bit by bit: one ballot and one v_bitop3 for each half of the mask.
+template <typename K, int U>
+__device__ __forceinline__ void rank_rows(const K (&k)[U], int pass, unsigned* mine, unsigned (&rank)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int d = digit_of(k[u], pass);
+        unsigned lo = ~0u, hi = ~0u;  // lanes with the same digit
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            int bit = __builtin_amdgcn_sbfe(d, b, 1);
+            asm("" : "+v"(bit));  // compared as it is, not shifted anew
+            const unsigned long long m = __ballot(bit != 0);
+            lo = __builtin_amdgcn_bitop3_b32(lo, (unsigned)m, (unsigned)bit, 0x90);  // lo & ~(m ^ bit)
+            hi = __builtin_amdgcn_bitop3_b32(hi, (unsigned)(m >> 32), (unsigned)bit, 0x90);
+        }
+        const unsigned ahead = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
+        rank[u] = ahead | (unsigned)(__popc(lo) + __popc(hi)) << 16;
+        // one row's masks at a time, and the test for a digit's first lane
+        // not before it is needed: 16 rows' masks would spill
+        asm volatile("" : "+v"(rank[u]));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        unsigned* const c = mine + digit_of(k[u], pass);
+        const unsigned before = *c, ahead = rank[u] & 0xFFFFu;
+        __builtin_amdgcn_wave_barrier();
+        if (ahead == 0) *c = before + (rank[u] >> 16);
+        __builtin_amdgcn_wave_barrier();
+        rank[u] = before + ahead;
+    }
+}
+
+// Thread t < 256: digit t's count in the tile (own), its keys' places before
+// each wave's (of_wave), and the sum of the lower digits' counts in t's wave
+// (upto) and, for all, in part[].
+template <int W>
+__device__ __forceinline__ void count_digits(const unsigned (&cnt)[W][kRadix], unsigned* part, unsigned& own,
+                                             unsigned& upto, unsigned (&of_wave)[W]) {
+    const int t = threadIdx.x, lane = t & 63;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+        of_wave[i] = own;
+        own += cnt[i][t];
+    }
+    upto = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned y = __shfl_up(upto, o, 64);
+        if (lane >= o) upto += y;
+    }
+    if (lane == 63) part[t >> 6] = upto;
+    upto -= own;
+}
+
 // One pass: the keys, in their present order, to the places their digit's
 // counts give.  Workgroups take tiles by ticket, so every tile before theirs
 // is finished or running and the look-back ends.
@@ -284,32 +362,36 @@ __device__ void copy_ascending(const BulkArgs<K>& a, const BulkPlan& pl) {
 //   * 256 threads, one per digit, publish the tile's counts and look back
 //     for those of the tiles before it; meanwhile the keys move into LDS in
 //     digit order, from where each digit's run is written as a whole.
+// What bounds it: vector instructions and LDS accesses (about 80 and 6 for 64
+// keys), at 2^28 u32 keys 850 us a pass, 2.5 TB/s read and written.  It took
+// 1150 us with lane masks built by selects (95 instructions for 64 keys; a
+// mask's step is one v_bitop3 now) and a look-back of one tile at a time,
+// each a round trip of about a microsecond.
 template <typename K>
 __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, int pass) {
     constexpr int T = bulk_tile<K>(), U = T / kBulkThreads, W = kBulkThreads / 64;
+    constexpr int kWindow = 16;  // tiles looked at together
     __shared__ K keys[T];
     __shared__ unsigned cnt[W][kRadix];
     __shared__ unsigned to[kRadix];
     __shared__ unsigned part[4];
     __shared__ int s_tile;
     const BulkPlan& pl = *a.mem.plan;
-    if (!pl.go) return;
-    if (pl.ascending) {
-        if (pass == 0) copy_ascending(a, pl);
-        return;
-    }
+    if (!pl.go || pl.ascending) return;
     const int ord = pl.order[pass];
     if (ord < 0) return;
     const bool first = ord == 0, last = ord == pl.active - 1;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int total = pl.total, tiles = pl.tiles;
     K* const spare = a.items + pl.spare;
-    const K* const src = (ord & 1) ? spare : a.items;
-    K* const dst = (ord & 1) ? a.items : spare;
+    K* const second = pl.through_out ? a.out + pl.off : a.items;
+    const K* const src = (ord & 1) ? spare : second;
+    // the last pass's places are not in a row where some keys stay
+    const bool split = last && !pl.drains;
+    K* const dst = last ? a.out + pl.off : (ord & 1) ? second : spare;
     unsigned* const look = a.mem.look[ord & 1];
     unsigned* const next = last ? nullptr : a.mem.look[(ord & 1) ^ 1];
     const unsigned start = t < kRadix ? a.mem.hist[pass * kRadix + t] : 0;
-    const unsigned long long below = (1ull << lane) - 1;
     for (;;) {
         if (t == 0) s_tile = (int)atomicAdd(a.mem.ticket + pass, 1u);
 #pragma unroll
@@ -325,49 +407,22 @@ __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, in
 #pragma unroll
             for (int u = 0; u < U; ++u) k[u] = run[j + u * 64];
         } else {
-#pragma unroll
+            // the last tile, and those across two parts of the source
+#pragma unroll 1
             for (int u = 0; u < U; ++u) {
                 const int i = j + u * 64;
-                k[u] = i < total ? (first ? *source_key(a, pl, i) : src[i]) : ~K(0);
+                keys[i - j0] = i < total ? *(first ? source_key(a, pl, i) : src + i) : ~K(0);
             }
+#pragma unroll
+            for (int u = 0; u < U; ++u) k[u] = keys[j - j0 + u * 64];  // a thread reads back its own
         }
-        // ranks among the wave's keys of the same digit (keys past the end
-        // count as digit 255 and come last)
-        unsigned short rank[U];
+        unsigned rank[U];
         unsigned* const mine = cnt[w];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int d = digit_of(k[u], pass);
-            unsigned long long same = ~0ull;
-#pragma unroll
-            for (int b = 0; b < 8; ++b) {
-                const bool bit = (d >> b) & 1;
-                const unsigned long long m = __ballot(bit);
-                same &= bit ? m : ~m;
-            }
-            const unsigned before = mine[d];
-            const int ahead = __popcll(same & below);
-            rank[u] = (unsigned short)(before + ahead);
-            __builtin_amdgcn_wave_barrier();
-            if (ahead == 0) mine[d] = before + __popcll(same);
-            __builtin_amdgcn_wave_barrier();
-        }
+        rank_rows(k, pass, mine, rank);
         __syncthreads();
         unsigned own = 0, upto = 0, of_wave[W];
         if (t < kRadix) {
-#pragma unroll
-            for (int i = 0; i < W; ++i) {
-                of_wave[i] = own;
-                own += cnt[i][t];
-            }
-            upto = own;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const unsigned y = __shfl_up(upto, o, 64);
-                if (lane >= o) upto += y;
-            }
-            if (lane == 63) part[w] = upto;
-            upto -= own;
+            count_digits(cnt, part, own, upto, of_wave);
             if (t == kRadix - 1) own -= T - here;  // padding does not count
             look_store(look + (size_t)tile * kRadix + t, (tile == 0 ? kLookAll : kLookOwn) | own);
             if (next) next[(size_t)tile * kRadix + t] = 0;
@@ -383,39 +438,61 @@ __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, in
         for (int u = 0; u < U; ++u) keys[mine[digit_of(k[u], pass)] + rank[u]] = k[u];
         unsigned before = 0;
         if (t < kRadix && tile > 0) {
-            const unsigned* p = look + (size_t)(tile - 1) * kRadix + t;
-            int polls = 0;
-            for (int back = tile - 1;;) {
-                const unsigned v = look_load(p);
-                if ((v >> 30) == 0) {
-                    // the tile before is running; the bound only ends a fault
-                    if (++polls > kSpinLimit) {
-                        __hip_atomic_fetch_or(a.ctr + CTR_ERROR * kWordStride, (int)ERR_SPIN_LIMIT, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-                        break;
+            const unsigned* const p = look + t;
+            int back = tile - 1, polls = 0;
+            for (bool open = true; open;) {
+                unsigned v[kWindow];
+#pragma unroll
+                for (int i = 0; i < kWindow; ++i)
+                    v[i] = look_load(p + (size_t)(back >= i ? back - i : 0) * kRadix);
+                bool ready = true;
+                const int at = back;
+#pragma unroll
+                for (int i = 0; i < kWindow; ++i) {
+                    ready = ready && (v[i] >> 30) != 0;
+                    if (ready && open) {
+                        before += v[i] & kLookCount;
+                        open = (v[i] >> 30) != 2;  // tile 0's count is of all
+                        --back;
                     }
-                    continue;
                 }
-                before += v & kLookCount;
-                if ((v >> 30) == 2 || back == 0) break;
-                --back;
-                p -= kRadix;
+                // the tile before is running; the bound only ends a fault
+                if (open && back == at && ++polls > kSpinLimit) {
+                    __hip_atomic_fetch_or(a.ctr + CTR_ERROR * kWordStride, (int)ERR_SPIN_LIMIT, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+                    break;
+                }
             }
             look_store(look + (size_t)tile * kRadix + t, kLookAll | (before + own));
         }
         if (t < kRadix) to[t] = start + before - upto;  // place of a key = to[digit] + its place in the tile
         __syncthreads();
+        if (here == T && !split) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int i = u * kBulkThreads + t;
-            if (i < here) {
+            for (int u = 0; u < U; ++u) {
+                const int i = u * kBulkThreads + t;
+                const K key = keys[i];
+                dst[to[digit_of(key, pass)] + (unsigned)i] = key;
+            }
+        } else {
+            for (int i = t; i < here; i += kBulkThreads) {
                 const K key = keys[i];
                 const int at = (int)to[digit_of(key, pass)] + i;
-                if (last) *final_place(a, pl, at) = key;
+                if (split) *final_place(a, pl, at) = key;
                 else dst[at] = key;
             }
         }
     }
+}
+
+// The heap's counters after a bulk call (one thread).
+template <typename K>
+__device__ __forceinline__ void set_counters(const BulkArgs<K>& a, const BulkPlan& pl) {
+    a.ctr[CTR_BATCH_COUNT * kWordStride] = pl.nb_after;
+    a.ctr[CTR_PARTIAL * kWordStride] = pl.pbs_after;
+    a.ctr[CTR_DELETE_COUNT * kWordStride] = pl.off + pl.cut;
+    a.ctr[CTR_ERROR * kWordStride] |= pl.error;
+    if (pl.idle && a.ctr[CTR_BUSY * kWordStride] <= 0) a.ctr[CTR_TERM * kWordStride] = 1;
 }
 
 // Batches that stay come back from the spare slots (ascending slots only);
@@ -447,27 +524,101 @@ __global__ __launch_bounds__(256) void k_bulk_finish(BulkArgs<K> a) {
     }
     if (!(pl.ascending && pl.pbs_after == pl.pbs))
         for (long long i = pl.pbs_after + i0; i < a.batch_size; i += step) a.items[i] = v;
-    if (i0 == 0) {
-        a.ctr[CTR_BATCH_COUNT * kWordStride] = pl.nb_after;
-        a.ctr[CTR_PARTIAL * kWordStride] = pl.pbs_after;
-        a.ctr[CTR_DELETE_COUNT * kWordStride] += pl.cut;
-        a.ctr[CTR_ERROR * kWordStride] |= pl.error;
-        if (pl.idle && a.ctr[CTR_BUSY * kWordStride] <= 0) a.ctr[CTR_TERM * kWordStride] = 1;
-    }
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < kSortWords; i += 256) a.mem.hist[i] = 0;
+    if (i0 == 0) set_counters(a, pl);
 }
+
+// A sort of one tile, whole: plan, passes in LDS, final places, counters.  The
+// free slots are not used.
+template <typename K>
+__global__ __launch_bounds__(kBulkThreads, 2) void k_bulk_tile(BulkArgs<K> a) {
+    constexpr int T = bulk_tile<K>(), U = T / kBulkThreads, W = kBulkThreads / 64, P = (int)sizeof(K);
+    __shared__ K keys[T];
+    __shared__ unsigned cnt[W][kRadix];
+    __shared__ unsigned part[4];
+    __shared__ BulkPlan pl;
+    const int t = threadIdx.x, w = t >> 6, j = w * (64 * U) + (t & 63);
+    if (t == 0) {
+        plan_insert(a, pl);
+        if (pl.total > T) pl.go = 0;
+        *a.mem.plan = pl;
+    }
+    __syncthreads();
+    if (!pl.go) return;
+    const int total = pl.total;
+    K k[U];
+#pragma unroll 1
+    for (int u = 0; u < U; ++u) keys[j + u * 64] = j + u * 64 < total ? *source_key(a, pl, j + u * 64) : ~K(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) k[u] = keys[j + u * 64];  // a thread reads back its own
+#pragma unroll 1
+    for (int pass = 0; pass < P; ++pass) {
+        unsigned rank[U];
+#pragma unroll
+        for (int i = 0; i < W * kRadix / kBulkThreads; ++i) (&cnt[0][0])[i * kBulkThreads + t] = 0;
+        __syncthreads();
+        rank_rows(k, pass, cnt[w], rank);
+        __syncthreads();
+        unsigned own = 0, upto = 0, of_wave[W];
+        if (t < kRadix) count_digits(cnt, part, own, upto, of_wave);
+        // (also the barrier before the sums and the counts are used)
+        if (__syncthreads_or(own == (unsigned)T)) continue;  // the digit is the same for all
+        if (t < kRadix) {
+            for (int i = 0; i < w; ++i) upto += part[i];
+#pragma unroll
+            for (int i = 0; i < W; ++i) cnt[i][t] = upto + of_wave[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < U; ++u) keys[cnt[w][digit_of(k[u], pass)] + rank[u]] = k[u];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < U; ++u) k[u] = keys[j + u * 64];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (j + u * 64 < total) *final_place(a, pl, j + u * 64) = k[u];
+    const long long used = (pl.nb + 1ll) * a.batch_size;
+    for (long long i = pl.fill_lo + t; i < used; i += kBulkThreads) a.items[i] = a.init_limits;
+    for (int i = pl.pbs_after + t; i < a.batch_size; i += kBulkThreads) a.items[i] = a.init_limits;
+    if (t == 0) set_counters(a, pl);
+}
+
+__global__ void k_bulk_report(const BulkPlan* pl, const int* ctr, int* report) {
+    const int i = threadIdx.x;
+    if (i <= CTR_WORDS) report[i] = i == 0 ? pl->go : ctr[(i - 1) * kWordStride];
+}
+static_assert(CTR_WORDS < kReportWords, "report words");
 
 inline int blocks_for(long long items, int per_block, int most) {
     const long long b = (items + per_block - 1) / per_block;
     return (int)(b < 1 ? 1 : (b > most ? most : b));
 }
 
+// The last kernel of every call; its end is the event `done`.
 template <typename K>
-hipError_t sort_and_finish(const BulkArgs<K>& a, long long keys, int cus, hipStream_t s) {
+void finish(const BulkArgs<K>& a, long long keys, hipEvent_t done, int cus, hipStream_t s) {
+    hipExtLaunchKernelGGL(k_bulk_finish<K>, dim3(blocks_for(keys, 4096, 8 * cus)), dim3(256), 0, s, nullptr, done, 0,
+                          a);
+}
+
+// The sort of about `keys` keys; `mid`, if any, is recorded before the pass of
+// the highest digit.
+template <typename K>
+hipError_t sort_and_finish(const BulkArgs<K>& a, long long keys, hipEvent_t mid, hipEvent_t done, int cus,
+                           hipStream_t s) {
+    constexpr int P = (int)sizeof(K);
     hipLaunchKernelGGL(k_bulk_hist<K>, dim3(blocks_for(keys, 4096, 4 * cus)), dim3(256), 0, s, a);
     const int grid = blocks_for(keys, bulk_tile<K>(), 3 * cus);
-    for (int p = 0; p < (int)sizeof(K); ++p)
+    for (int p = 0; p < P; ++p) {
+        if (p == P - 1 && mid) {
+            const hipError_t e = hipEventRecord(mid, s);
+            if (e != hipSuccess) return e;
+        }
         hipLaunchKernelGGL(k_bulk_pass<K>, dim3(grid), dim3(kBulkThreads), 0, s, a, p);
-    hipLaunchKernelGGL(k_bulk_finish<K>, dim3(blocks_for(keys, 4096, 8 * cus)), dim3(256), 0, s, a);
+    }
+    finish(a, keys, done, cus, s);
     return hipGetLastError();
 }
 
@@ -485,39 +636,62 @@ BulkArgs<K> args_for(const bgpq_heap* h) {
 
 template <typename K>
 hipError_t insert_as(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap, long long calls,
-                     int cus, hipStream_t s) {
+                     hipEvent_t mid, int cus, hipStream_t s) {
     BulkArgs<K> a = args_for<K>(h);
     a.keys = (const K*)keys;
     a.n = n;
     a.out = (K*)out;
     a.out_cap = out_cap;
     a.calls = calls;
+    a.from_empty = mid != nullptr;
     clear_last_error();
-    hipLaunchKernelGGL(k_plan_insert<K>, dim3(1), dim3(256), 0, s, a);
-    return sort_and_finish(a, h->held + n, cus, s);
+    if (bulk_one_tile(h, h->held + n)) {
+        if (mid) {
+            const hipError_t e = hipEventRecord(mid, s);
+            if (e != hipSuccess) return e;
+        }
+        hipExtLaunchKernelGGL(k_bulk_tile<K>, dim3(1), dim3(kBulkThreads), 0, s, nullptr, h->bulk_done, 0, a);
+        return hipGetLastError();
+    }
+    return sort_and_finish(a, h->held + n, mid, h->bulk_done, cus, s);
 }
 
 template <typename K>
-hipError_t delete_as(const bgpq_heap* h, void* out, long long out_cap, long long calls, int cus, hipStream_t s) {
+hipError_t delete_as(const bgpq_heap* h, void* out, long long out_cap, long long calls, bool ascends, int cus,
+                     hipStream_t s) {
     BulkArgs<K> a = args_for<K>(h);
     a.out = (K*)out;
     a.out_cap = out_cap;
     a.calls = calls;
+    a.planned = 1;
+    a.sorts = !ascends;
     clear_last_error();
     hipLaunchKernelGGL(k_plan_delete<K>, dim3(blocks_for(h->held / h->batch_size, 256, cus)), dim3(256), 0, s, a);
-    return sort_and_finish(a, h->held, cus, s);
+    hipLaunchKernelGGL(k_bulk_copy<K>, dim3(blocks_for(h->held, 8 * kBulkThreads, 4 * cus)), dim3(kBulkThreads), 0, s,
+                       a);
+    if (!ascends) return sort_and_finish(a, h->held, nullptr, h->bulk_done, cus, s);
+    finish(a, h->held, h->bulk_done, cus, s);
+    return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap,
-                       long long calls, int cus, hipStream_t s) {
-    return h->key_type == BGPQ_KEY_U64 ? insert_as<uint64_t>(h, keys, n, out, out_cap, calls, cus, s)
-                                       : insert_as<uint32_t>(h, keys, n, out, out_cap, calls, cus, s);
+                       long long calls, hipEvent_t mid, int cus, hipStream_t s) {
+    return h->key_type == BGPQ_KEY_U64 ? insert_as<uint64_t>(h, keys, n, out, out_cap, calls, mid, cus, s)
+                                       : insert_as<uint32_t>(h, keys, n, out, out_cap, calls, mid, cus, s);
 }
-hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, int cus, hipStream_t s) {
-    return h->key_type == BGPQ_KEY_U64 ? delete_as<uint64_t>(h, out, out_cap, calls, cus, s)
-                                       : delete_as<uint32_t>(h, out, out_cap, calls, cus, s);
+bool bulk_one_tile(const bgpq_heap* h, long long keys) {
+    return keys <= (h->key_type == BGPQ_KEY_U64 ? bulk_tile<uint64_t>() : bulk_tile<uint32_t>());
+}
+hipError_t bulk_report(const bgpq_heap* h, int* report, hipStream_t s) {
+    hipLaunchKernelGGL(k_bulk_report, dim3(1), dim3(64), 0, s, h->bulk.plan, h->ctr, report);
+    return hipGetLastError();
+}
+hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, bool ascends, int cus,
+                       hipStream_t s) {
+    return h->key_type == BGPQ_KEY_U64 ? delete_as<uint64_t>(h, out, out_cap, calls, ascends, cus, s)
+                                       : delete_as<uint32_t>(h, out, out_cap, calls, ascends, cus, s);
 }
 
 }  // namespace bgpq

@@ -26,8 +26,11 @@ namespace bgpq {
 constexpr int kRadix = 256;        // 8-bit digits
 constexpr int kMaxPasses = 8;      // of a u64 key
 constexpr int kBulkThreads = 512;  // of a pass's workgroup (8 waves)
-// Keys a workgroup takes at a time: 32 KB of LDS, which with the counters
-// leaves room for 3 workgroups on a CU.
+// Keys a workgroup takes at a time (a tile): 32 KB of LDS, which with the
+// counters leaves room for 3 workgroups on a CU.  Smaller tiles are no faster
+// even where these leave CUs idle, since the look-back gets longer (2^20 u32
+// keys: 159, 163, 182 us with 8192, 4096, 2048 keys a tile; u64 rounds of
+// 1.5 M keys in all: 983, 1103, 1415 us with 4096, 2048, 1024).
 template <typename K>
 constexpr int bulk_tile() { return 32768 / (int)sizeof(K); }
 // Above this the lookback words' 30-bit counts would not do.
@@ -37,6 +40,7 @@ constexpr long long kBulkMaxKeys = 1ll << 30;
 struct BulkPlan {
     int go;               // 0: the per-batch kernel runs instead
     int ascending;        // delete: the slots already ascend, no sort needed
+    int drains;           // every key is handed out
     int nb, pbs;          // batches and partial keys found
     int total;            // keys sorted
     int tiles;
@@ -50,17 +54,23 @@ struct BulkPlan {
     int idle;             // a deletion found nothing (termination vote)
     int active;           // passes that move keys
     int order[kMaxPasses];  // position of a pass among them, -1: skipped
-    int violations, arrived;  // working words, 0 between calls
+    int through_out;        // the passes alternate between the free slots and the output
 };
 
-// Device memory of a handle's bulk calls.
+// Device memory of a handle's bulk calls.  The sort words (hist, ticket,
+// sync) are 0 between calls.
 struct BulkMem {
     BulkPlan* plan;
     unsigned* hist;      // [kMaxPasses][kRadix] key counts, then first positions
     unsigned* ticket;    // [kMaxPasses] next tile of a pass
+    int* sync;           // violations found, workgroups arrived
     unsigned* look[2];   // [tiles][kRadix] lookback words, alternating by pass
     int tiles_max;
 };
+// What a heap sort's end tells the host (pinned memory): the plan's `go` and
+// the counter words.
+constexpr int kReportWords = 16;
+constexpr int kSortWords = kMaxPasses * (kRadix + 1) + 2;
 
 // One bulk call on one heap.
 template <typename K>
@@ -73,6 +83,9 @@ struct BulkArgs {
     long long n;
     K* out;         // popped, by `calls` deletions
     long long out_cap, calls;
+    int from_empty; // only on an empty heap, the output from its start
+    int planned;    // the plan is in memory already (k_plan_delete)
+    int sorts;      // the sort's kernels follow, not the copy of ascending slots
     BulkMem mem;
 };
 

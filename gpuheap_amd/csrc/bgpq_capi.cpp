@@ -72,8 +72,8 @@ static HeapArgs args_of(const bgpq_heap* h, long long out_cap = 0) {
 }
 
 // The bulk calls' words follow the counters and, for their lookback, the
-// slots, in the same allocations.  Lookback words are there for the most keys
-// a bulk sort can take: their slots and as many free ones.
+// slots, in the same allocations.  Lookback words are there for the most tiles
+// a bulk sort can have: of keys that take half the slots.
 static size_t items_bytes(const bgpq_heap* h) {
     return key_bytes(h->key_type) * (size_t)h->batch_size * (size_t)(h->batch_num + 1);
 }
@@ -84,7 +84,7 @@ static int bulk_tiles_max(const bgpq_heap* h) {
     return (int)(keys / tile + 1);
 }
 static size_t bulk_fixed_bytes() {
-    return up256(ctr_bytes()) + up256(sizeof(BulkPlan)) + up256(sizeof(unsigned) * kMaxPasses * (kRadix + 1));
+    return up256(ctr_bytes()) + up256(sizeof(BulkPlan)) + up256(sizeof(unsigned) * kSortWords);
 }
 static size_t bulk_look_bytes(const bgpq_heap* h) { return sizeof(unsigned) * kRadix * (size_t)bulk_tiles_max(h); }
 static void set_bulk_mem(bgpq_heap* h) {
@@ -93,12 +93,12 @@ static void set_bulk_mem(bgpq_heap* h) {
     p += up256(sizeof(BulkPlan));
     h->bulk.hist = (unsigned*)p;
     h->bulk.ticket = h->bulk.hist + kMaxPasses * kRadix;
+    h->bulk.sync = (int*)(h->bulk.ticket + kMaxPasses);
     p = (char*)h->items + up256(items_bytes(h));
     h->bulk.look[0] = (unsigned*)p;
     h->bulk.look[1] = (unsigned*)(p + bulk_look_bytes(h));
     h->bulk.tiles_max = bulk_tiles_max(h);
 }
-
 
 static int fill_items(bgpq_heap* h, hipStream_t s) {
     const long long n = (long long)(h->batch_num + 1) * h->batch_size;
@@ -123,16 +123,26 @@ static bool capturing(hipStream_t s) {
     return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
 
+// The bulk calls end for good once work may run beside them: calls on a second
+// stream, or captured ones, whose graph may run at any time.
 int bgpq_on_stream(bgpq_heap* h, hipStream_t s) {
-    if (h->used && s != h->stream) {
+    std::lock_guard<std::recursive_mutex> hold(h->lock);
+    const bool captured = capturing(s);
+    if (captured || (h->used && s != h->stream)) {
         h->shared = true;
-        if (h->bulk_open && !capturing(s)) {
-            HIPCHK(hipDeviceSynchronize());
+        if (h->bulk_open) {
+            // other streams' events may be waited for while this thread captures
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            if (captured) (void)hipThreadExchangeStreamCaptureMode(&mode);
+            const hipError_t e = hipEventSynchronize(h->bulk_done);
+            if (captured) (void)hipThreadExchangeStreamCaptureMode(&mode);
+            if (e != hipSuccess) return fail(BGPQ_EHIP, "wait for the last bulk call: %s", hipGetErrorString(e));
             h->bulk_open = false;
         }
     }
     h->used = true;
     h->stream = s;
+    h->ascends = false;
     return BGPQ_OK;
 }
 
@@ -265,11 +275,16 @@ void bgpq_destroy(bgpq_heap* h) {
     if (h->status) (void)hipFree(h->status);
     if (h->ctr) (void)hipFree(h->ctr);
     if (h->app_ctl) (void)hipFree(h->app_ctl);
+    if (h->bulk_done) (void)hipEventDestroy(h->bulk_done);
+    for (hipEvent_t e : h->sort_events)
+        if (e) (void)hipEventDestroy(e);
+    if (h->sort_report) (void)hipHostFree(h->sort_report);
     delete h;
 }
 
 int bgpq_reset(bgpq_heap* h, void* stream) {
     if (!h) return fail(BGPQ_EINVAL, "null handle");
+    std::lock_guard<std::recursive_mutex> hold(h->lock);
     const int rc = bgpq_on_stream(h, (hipStream_t)stream);
     if (rc) return rc;
     h->held = 0;
@@ -315,6 +330,7 @@ int bgpq_terminated(bgpq_heap* h) {
 int bgpq_clear(bgpq_heap* h, void* stream) {
     if (!h) return fail(BGPQ_EINVAL, "null handle");
     hipStream_t s = (hipStream_t)stream;
+    std::lock_guard<std::recursive_mutex> hold(h->lock);
     const int rc = bgpq_on_stream(h, s);
     if (rc) return rc;
     h->held = 0;
@@ -407,57 +423,66 @@ static int resolve_grid(bgpq_heap* h, int grid) { return grid > 0 ? grid : bgpq_
 
 static bool np_variant(const bgpq_heap* h) { return h->variant == BGPQ_BUITDD_NP || h->variant == BGPQ_TDITDD_NP; }
 
-// Whether `calls` insertions or pops are done together (bgpq_bulk.hpp):
-// where one after the other, at `each` us apart, would take longer than the
-// bulk kernels' launches (about 60 us) and their passes over the heap's
-// `keys` keys (u32 keys of 4 passes 16 ps each, u64 keys of 8 passes 50 ps).
-// Heap sort of 2^20 u32 keys, B = 1024: 7590 us one by one, 170 us together;
-// of 2^28, B = 8192: 367 ms and 6.6 ms; of 3 M u64 keys, B = 1024: 39.9 ms
-// and 0.41 ms.
-static bool bulk_pays(const bgpq_heap* h, long long calls, double each, long long keys) {
-    const double per_key = h->key_type == BGPQ_KEY_U64 ? 50e-6 : 16e-6;
-    return keys < kBulkMaxKeys && calls * each > 60.0 + keys * per_key;
+// Whether calls are done together (bgpq_bulk.hpp): where one after the other
+// they would take longer.  An insertion takes 2 us and a pop 4 at the least
+// (B = 256), whatever the grid; a bulk call takes its launches, 60 us with a
+// sort, 30 with one of one tile, 20 from slots that ascend, and its passes
+// over the heap's `keys` keys (u32 keys of 4 passes 15 ps each, u64 keys of 8
+// passes 50 ps).
+static double sort_us(const bgpq_heap* h, long long keys, bool one = false) {
+    if (one && bulk_one_tile(h, keys)) return 30.0;
+    return 60.0 + keys * (h->key_type == BGPQ_KEY_U64 ? 50e-6 : 15e-6);
+}
+static bool insert_pays(const bgpq_heap* h, long long calls, long long keys) {
+    return keys < kBulkMaxKeys && calls * 2.0 > sort_us(h, keys, true);
+}
+static bool delete_pays(const bgpq_heap* h, long long calls, long long keys, bool ascends) {
+    return keys < kBulkMaxKeys && calls * 4.0 > (ascends ? 20.0 + keys * 5e-6 : sort_us(h, keys));
+}
+static bool sort_pays(const bgpq_heap* h, long long in, long long pops, long long keys) {
+    return keys < kBulkMaxKeys && in * 2.0 + pops * 4.0 > sort_us(h, keys, true);
 }
 
 // A grid of one workgroup keeps the calls' own order, one after the other;
 // keys that are not aligned to their size only the per-batch kernels take.
-static bool bulk_can(const bgpq_heap* h, const void* keys, int grid, hipStream_t s) {
-    return !h->shared && grid != 1 && s != hipStreamPerThread && (uintptr_t)keys % key_bytes(h->key_type) == 0 &&
-           !capturing(s);
+static bool bulk_can(bgpq_heap* h, const void* keys, int grid, hipStream_t s) {
+    if (h->shared || grid == 1 || s == hipStreamPerThread || (uintptr_t)keys % key_bytes(h->key_type) != 0)
+        return false;
+    return h->bulk_done || hipEventCreateWithFlags(&h->bulk_done, hipEventDisableTiming) == hipSuccess;
 }
 
-// `sure`: the caller has seen that the plan cannot refuse.
-static int insert_calls(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, int grid, hipStream_t s, bool sure) {
+static int insert_calls(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, int grid, hipStream_t s) {
+    std::lock_guard<std::recursive_mutex> hold(h->lock);
     const int rc = bgpq_on_stream(h, s);
     if (rc) return rc;
     HeapArgs a = args_of(h);
-    if (bulk_pays(h, (n + chunk - 1) / chunk, 2.0, h->held + n) && bulk_can(h, d_keys, grid, s)) {
-        const hipError_t e = bulk_insert(h, d_keys, n, nullptr, 0, 0, bgpq_default_grid(h->batch_size), s);
+    if (insert_pays(h, (n + chunk - 1) / chunk, h->held + n) && bulk_can(h, d_keys, grid, s)) {
+        const hipError_t e = bulk_insert(h, d_keys, n, nullptr, 0, 0, nullptr, bgpq_default_grid(h->batch_size), s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk insert launch: %s", hipGetErrorString(e));
-        h->bulk_open = true;
+        h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
     }
     h->held += n;
-    if (a.skip && sure) return BGPQ_OK;
     const hipError_t e = h->row->insert(a, d_keys, n, chunk, resolve_grid(h, grid), s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "insert launch: %s", hipGetErrorString(e));
     return BGPQ_OK;
 }
 
-static int delete_calls(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t calls, int grid, hipStream_t s,
-                        bool sure) {
+static int delete_calls(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t calls, int grid, hipStream_t s) {
+    std::lock_guard<std::recursive_mutex> hold(h->lock);
+    const bool ascends = h->ascends;
     const int rc = bgpq_on_stream(h, s);
     if (rc) return rc;
     HeapArgs a = args_of(h, out_keys);
     const long long pops = std::min<long long>(calls, (h->held + h->batch_size - 1) / h->batch_size);
-    if (bulk_pays(h, pops, 4.0, h->held) && bulk_can(h, d_out, grid, s)) {
-        const hipError_t e = bulk_delete(h, d_out, out_keys, calls, bgpq_default_grid(h->batch_size), s);
+    if (delete_pays(h, pops, h->held, ascends) && bulk_can(h, d_out, grid, s)) {
+        const hipError_t e =
+            bulk_delete(h, d_out, out_keys, calls, ascends, bgpq_default_grid(h->batch_size), s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk delete launch: %s", hipGetErrorString(e));
-        h->bulk_open = true;
+        h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
     }
     h->held = std::max<long long>(h->held - pops * h->batch_size, 0);
-    if (a.skip && sure) return BGPQ_OK;
     const hipError_t e = h->row->del(a, d_out, calls, resolve_grid(h, grid), s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "delete launch: %s", hipGetErrorString(e));
     return BGPQ_OK;
@@ -472,7 +497,7 @@ int bgpq_insert(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, int grid
     if (chunk > h->batch_size) return fail(BGPQ_EINVAL, "chunk %d > batch size %d", chunk, h->batch_size);
     if (np_variant(h) && (chunk != h->batch_size || n % h->batch_size))
         return fail(BGPQ_EINVAL, "_np variants insert full batches only (chunk %d, n %lld)", chunk, (long long)n);
-    return insert_calls(h, d_keys, n, chunk, grid, (hipStream_t)stream, false);
+    return insert_calls(h, d_keys, n, chunk, grid, (hipStream_t)stream);
 }
 
 int bgpq_delete(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t calls, int grid, void* stream) {
@@ -481,7 +506,7 @@ int bgpq_delete(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t calls, int 
                                                (long long)out_keys);
     if (calls == 0) return BGPQ_OK;
     if (!d_out) return fail(BGPQ_EINVAL, "null output");
-    return delete_calls(h, d_out, out_keys, calls, grid, (hipStream_t)stream, false);
+    return delete_calls(h, d_out, out_keys, calls, grid, (hipStream_t)stream);
 }
 
 int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chunk, void* d_out, int64_t out_keys,
@@ -497,6 +522,7 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
     if ((n_insert && !d_keys) || (calls && !d_out)) return fail(BGPQ_EINVAL, "null buffer");
     if (out_keys < 0) return fail(BGPQ_EINVAL, "out_keys %lld", (long long)out_keys);
     hipStream_t s = (hipStream_t)stream;
+    std::lock_guard<std::recursive_mutex> hold(h->lock);
     const int rc = bgpq_on_stream(h, s);
     if (rc) return rc;
     HeapArgs a = args_of(h, out_keys);
@@ -504,16 +530,45 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
     // the concurrent kernel may take
     const long long in = (n_insert + chunk - 1) / chunk, all = h->held + n_insert;
     const long long pops = std::min<long long>(calls, (all + h->batch_size - 1) / h->batch_size);
-    if (bulk_pays(h, in + pops, 3.0, all) && bulk_can(h, d_keys, grid, s) && bulk_can(h, d_out, grid, s)) {
+    if (sort_pays(h, in, pops, all) && bulk_can(h, d_keys, grid, s) && bulk_can(h, d_out, grid, s)) {
         const hipError_t e =
-            bulk_insert(h, d_keys, n_insert, d_out, out_keys, calls, bgpq_default_grid(h->batch_size), s);
+            bulk_insert(h, d_keys, n_insert, d_out, out_keys, calls, nullptr, bgpq_default_grid(h->batch_size), s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk launch: %s", hipGetErrorString(e));
-        h->bulk_open = true;
+        h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
     }
     h->held = std::max<long long>(all - pops * h->batch_size, 0);
     hipError_t e = h->row->conc(a, d_keys, n_insert, chunk, d_out, calls, grid, s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "concurrent launch: %s", hipGetErrorString(e));
+    return BGPQ_OK;
+}
+
+// A heap sort as one bulk call: both halves are one sort, and the pass of the
+// highest digit, which hands the keys out, counts as the second.  *done is
+// false where the heap turned out not to be empty or is aborted: the caller
+// goes on as if the call had not been made.  Nothing is asked of the device
+// before or between (of 150 us for 2^20 u32 keys, 60 were two copies of the
+// counters, a memset and the making of events).
+static int bulk_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n, int64_t pops, float* ms_insert,
+                         float* ms_delete, hipStream_t s, bool* done) {
+    hipEvent_t* const ev = h->sort_events;
+    HIPCHK(hipEventRecord(ev[0], s));
+    const hipError_t e = bulk_insert(h, d_in, n, d_out, n, pops + 1, ev[1], bgpq_default_grid(h->batch_size), s);
+    if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk launch: %s", hipGetErrorString(e));
+    h->bulk_open = h->ascends = true;
+    HIPCHK(hipEventRecord(ev[2], s));
+    const hipError_t r = bulk_report(h, h->sort_report, s);
+    if (r != hipSuccess) return fail(BGPQ_EHIP, "report launch: %s", hipGetErrorString(r));
+    HIPCHK(hipStreamSynchronize(s));
+    *done = h->sort_report[0] != 0;
+    if (!*done) return BGPQ_OK;
+    float a = 0, b = 0;
+    HIPCHK(hipEventElapsedTime(&a, ev[0], ev[1]));
+    HIPCHK(hipEventElapsedTime(&b, ev[1], ev[2]));
+    if (ms_insert) *ms_insert = a;
+    if (ms_delete) *ms_delete = b;
+    const int error = h->sort_report[1 + CTR_ERROR];
+    if (error) return fail(BGPQ_EHEAP, "device error flags 0x%x", error);
     return BGPQ_OK;
 }
 
@@ -524,50 +579,49 @@ int bgpq_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n, int ch
     if (n > 0x7FFFFFFF) return fail(BGPQ_EINVAL, "the heap-sort cursor is 32-bit: n <= 2^31-1");
     hipStream_t s = (hipStream_t)stream;
     if (chunk <= 0) chunk = h->batch_size;
+    std::lock_guard<std::recursive_mutex> hold(h->lock);
     int rc = bgpq_on_stream(h, s);
     if (rc) return rc;
+    const int64_t B = h->batch_size, in = (n + chunk - 1) / chunk, pops = (n + B - 1) / B;
+    const bool fits = pops <= (int64_t)h->batch_num / 2;
+    const bool whole = !np_variant(h) || n == 0 || (chunk == h->batch_size && n % B == 0);
+    hipEvent_t* const ev = h->sort_events;
+    for (int i = 0; i < 3; ++i)
+        if (!ev[i]) HIPCHK(hipEventCreate(&ev[i]));
+    if (h->held == 0 && fits && chunk <= h->batch_size && whole && sort_pays(h, in, pops, n) &&
+        bulk_can(h, d_in, grid_insert, s) && bulk_can(h, d_out, grid_delete, s)) {
+        if (!h->sort_report) HIPCHK(hipHostMalloc((void**)&h->sort_report, kReportWords * sizeof(int), 0));
+        bool done = false;
+        rc = bulk_heapsort(h, d_in, d_out, n, pops, ms_insert, ms_delete, s, &done);
+        if (rc || done) return rc;
+    }
     int c[CTR_WORDS];
     rc = counters(h, c);
     if (rc) return rc;
-    const int64_t items = h->held;
-    if (items != 0) return fail(BGPQ_EINVAL, "heap sort needs an empty heap (%lld items)", (long long)items);
-    const int64_t B = h->batch_size;
-    if ((n + B - 1) / B > (int64_t)h->batch_num / 2)
+    if (h->held != 0) return fail(BGPQ_EINVAL, "heap sort needs an empty heap (%lld items)", h->held);
+    if (!fits)
         return fail(BGPQ_EINVAL, "capacity: %lld keys need batch_num >= %lld", (long long)n,
                     (long long)(2 * ((n + B - 1) / B)));
     if (chunk > h->batch_size) return fail(BGPQ_EINVAL, "chunk %d > batch size %d", chunk, h->batch_size);
-    if (np_variant(h) && n > 0 && (chunk != h->batch_size || n % h->batch_size))
+    if (!whole)
         return fail(BGPQ_EINVAL, "_np variants insert full batches only (chunk %d, n %lld)", chunk, (long long)n);
-    // the heap is empty and the keys fit twice: only an aborted heap makes
-    // a bulk call refuse
-    const bool sure = c[CTR_ABORT] == 0;
     HIPCHK(hipMemsetAsync(h->ctr + CTR_DELETE_COUNT * kWordStride, 0, sizeof(int), s));
-    hipEvent_t e0, e1, e2;
-    HIPCHK(hipEventCreate(&e0));
-    HIPCHK(hipEventCreate(&e1));
-    HIPCHK(hipEventCreate(&e2));
-    HIPCHK(hipEventRecord(e0, s));
-    if (n > 0) rc = insert_calls(h, d_in, n, chunk, grid_insert, s, sure);
-    if (!rc) {
-        HIPCHK(hipEventRecord(e1, s));
-        // enough calls to drain: every call removes a full batch or the partial buffer
-        if (d_out) rc = delete_calls(h, d_out, n, (n + B - 1) / B + 1, grid_delete, s, sure);
-        else rc = fail(BGPQ_EINVAL, "null output");
-    }
-    if (!rc) {
-        HIPCHK(hipEventRecord(e2, s));
-        HIPCHK(hipEventSynchronize(e2));
-        float a = 0, b = 0;
-        HIPCHK(hipEventElapsedTime(&a, e0, e1));
-        HIPCHK(hipEventElapsedTime(&b, e1, e2));
-        if (ms_insert) *ms_insert = a;
-        if (ms_delete) *ms_delete = b;
-        rc = device_error(h);
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    (void)hipEventDestroy(e2);
-    return rc;
+    HIPCHK(hipEventRecord(ev[0], s));
+    if (n > 0) rc = insert_calls(h, d_in, n, chunk, grid_insert, s);
+    if (rc) return rc;
+    HIPCHK(hipEventRecord(ev[1], s));
+    if (!d_out) return fail(BGPQ_EINVAL, "null output");
+    // enough calls to drain: every call removes a full batch or the partial buffer
+    rc = delete_calls(h, d_out, n, pops + 1, grid_delete, s);
+    if (rc) return rc;
+    HIPCHK(hipEventRecord(ev[2], s));
+    HIPCHK(hipEventSynchronize(ev[2]));
+    float a = 0, b = 0;
+    HIPCHK(hipEventElapsedTime(&a, ev[0], ev[1]));
+    HIPCHK(hipEventElapsedTime(&b, ev[1], ev[2]));
+    if (ms_insert) *ms_insert = a;
+    if (ms_delete) *ms_delete = b;
+    return device_error(h);
 }
 
 int bgpq_test_sort(int key_type, int batch_size, const void* d_in, const int* d_sizes, void* d_out,

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
+
 #include "bgpq.h"
 #include "bgpq_bulk.hpp"
 #include "bgpq_kernels.hpp"
@@ -30,21 +32,40 @@ struct bgpq_heap {
     bool shared;
     bool used;           // a call was made, on `stream`
     hipStream_t stream;
-    hipEvent_t bulk_done;  // end of the last bulk call, for calls on other streams
-    bool bulk_open;
+    hipEvent_t bulk_done;  // end of the last bulk call, made with the first
+    bool bulk_open;        // calls on another stream have to wait for it
+    bool ascends;          // like `held`: the last call was a bulk call
+    // A heap sort's start, middle and end, and what its end tells the host;
+    // made with the first one.
+    hipEvent_t sort_events[3];
+    int* sort_report;
+    // Held while a call's kernels are put on its stream: a bulk call's
+    // kernels must not mix with those of another thread's call.
+    std::recursive_mutex lock;
 };
 
 // To be called before work of the heap is put on a stream: notes the stream
-// and, where the stream changes, waits for a bulk call on the last one.
+// and, where it changes or is captured, ends the bulk calls and waits for the
+// last one.
 int bgpq_on_stream(bgpq_heap* h, hipStream_t s);
 
 namespace bgpq {
 // The launch sequences of bgpq_bulk.hip.  A per-batch kernel with
 // HeapArgs::skip = &plan->go must follow them, unless the plan cannot refuse.
-// bulk_insert: n keys in, then `calls` deletions (0 for none).
+// bulk_insert: n keys in, then `calls` deletions (0 for none).  With `mid` a
+// heap sort: refused unless the heap is empty, the output starts at its first
+// key whatever the cursor, and `mid` is recorded before the pass of the
+// highest digit.
+// bulk_report: kReportWords words of pinned memory, behind a heap sort.
+// bulk_delete: `ascends` where the slots are expected to ascend (a plan that
+// finds otherwise refuses).
 hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap,
-                       long long calls, int cus, hipStream_t s);
-hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, int cus, hipStream_t s);
+                       long long calls, hipEvent_t mid, int cus, hipStream_t s);
+// Whether an insertion that makes `keys` keys in all is sorted by one workgroup.
+bool bulk_one_tile(const bgpq_heap* h, long long keys);
+hipError_t bulk_report(const bgpq_heap* h, int* report, hipStream_t s);
+hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, bool ascends, int cus,
+                       hipStream_t s);
 }  // namespace bgpq
 
 // Records the message returned by bgpq_last_error and returns `code`.

@@ -201,6 +201,39 @@ def test_bulk_limits(gpu, variant):
         h.close()
 
 
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("key", ["u32", "u64"])
+@pytest.mark.parametrize("order", ["random", "ties", "one", "byte2"])
+def test_bulk_one_tile(gpu, variant, key, order):
+    """Calls of one workgroup's sort (8192 u32, 4096 u64 keys and fewer): heap
+    sorts of odd sizes around it, insertions into a heap that holds keys, and
+    concurrent calls that leave some."""
+    B, tile = 64, 8192 if key == "u32" else 4096
+    for n in (20 * B, 20 * B + 1, tile - 1, tile, tile + 1):
+        n = n if variant in PB else n // B * B
+        print(f"[case] one tile {variant} {key} {order} n={n}", flush=True)
+        keys = _keys(key, n, n, order)
+        h = Heap(batch_num_for(n, B) + 64, B, variant=variant, key=key)
+        d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer(keys.nbytes)
+        h.heapsort(d, n, d_out=out)
+        assert np.array_equal(out.to_numpy(keys.dtype, n), np.sort(keys))
+        _valid(h, keys[:0])
+        h.insert(d, 19 * B)  # a bulk call, then more beside the keys held
+        _valid(h, keys[:19 * B])
+        h.set_cursor(0)
+        m = n - 19 * B
+        h.concurrent(d.ptr + 19 * B * keys.itemsize, m, out, 12, chunk=B)
+        G.sync()
+        done = int(h.snapshot()[2][2])
+        assert done == min(12, n // B) * B
+        if m // B >= 4:  # enough calls to be done together
+            assert np.array_equal(out.to_numpy(keys.dtype, done), np.sort(keys)[:done])
+            _valid(h, np.sort(keys)[done:])
+        with pytest.raises(G.BgpqError, match="empty heap"):
+            h.heapsort(d, B, d_out=out)
+        h.close()
+
+
 def test_bulk_needs_the_heap_to_itself(gpu):
     """After its view was handed out a heap takes the per-batch kernels only:
     the words of a walked heap differ from the ascending layout."""
