@@ -18,10 +18,17 @@ __global__ __launch_bounds__(threads_for(B)) void k_sssp(HeapView<uint64_t> h, S
                                                          uint64_t first) {
     drive<VAR, B, threads_for(B)>(h, app, ctl, first, blockIdx.x == 0, (int)gridDim.x);
 }
+// An A* solve is a chain of pops, each a step further along the path, so what
+// counts is one workgroup's loop: a thread a key, where the heap's kernels
+// hold two (1024^2 cells, B = 256, 4 workgroups: 26.4 -> 23.6 ms, expansions
+// 8.5 -> 7.2 us a loop and the sift's merges shorter).  With more threads the
+// other drivers, whose workgroups wait for each other, are no faster
+// (knapsack of 200 items 13.6 -> 14.0 ms).
+constexpr int astar_threads(int B) { return B <= 512 ? B : threads_for(B); }
 template <int VAR, int B>
-__global__ __launch_bounds__(threads_for(B)) void k_astar(HeapView<uint64_t> h, AstarApp app, long long* ctl,
-                                                          uint64_t first) {
-    drive<VAR, B, threads_for(B)>(h, app, ctl, first, blockIdx.x == 0, (int)gridDim.x);
+__global__ __launch_bounds__(astar_threads(B)) void k_astar(HeapView<uint64_t> h, AstarApp app, long long* ctl,
+                                                            uint64_t first) {
+    drive<VAR, B, astar_threads(B)>(h, app, ctl, first, blockIdx.x == 0, (int)gridDim.x);
 }
 template <int VAR, int B>
 __global__ __launch_bounds__(threads_for(B)) void k_knapsack(HeapView<uint64_t> h, KnapsackApp app,
@@ -75,7 +82,7 @@ struct AppRows {
         static const hipError_t ok = prep(&k_astar<VAR, B>);
         if (ok != hipSuccess) return ok;
         (void)hipGetLastError();
-        hipLaunchKernelGGL((k_astar<VAR, B>), dim3(grid), dim3(threads_for(B)), lds, s, view_of<uint64_t>(a), app,
+        hipLaunchKernelGGL((k_astar<VAR, B>), dim3(grid), dim3(astar_threads(B)), lds, s, view_of<uint64_t>(a), app,
                            ctl, first);
         return hipGetLastError();
     }

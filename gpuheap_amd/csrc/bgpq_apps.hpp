@@ -91,6 +91,9 @@ __device__ __forceinline__ uint32_t u32_max(uint32_t* p, uint32_t v) {
 __device__ __forceinline__ uint64_t u64_load(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void u64_store(uint64_t* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // Exclusive prefix sum over the workgroup; `tmp` holds NT/64 values.
 template <int NT, typename T>
@@ -538,9 +541,12 @@ struct KnapsackApp {
     long long pool_cap;
     long long* ctl;
 
+    // (In words: a 16-byte buffer load of a place that differs from lane to
+    // lane is a loop over the lanes, 10 us for a wave's records.)
     __device__ KnapNode load_node(uint32_t idx) const {
-        const uint4 q = gload16(buf_rsrc(pool + idx), 0);
-        return KnapNode{q.x, q.y, q.z, q.w};
+        const uint64_t* q = reinterpret_cast<const uint64_t*>(pool + idx);
+        const uint64_t a = u64_load(q), b = u64_load(q + 1);
+        return KnapNode{(uint32_t)a, (uint32_t)(a >> 32), (uint32_t)b, (uint32_t)(b >> 32)};
     }
     __device__ uint32_t* slot(uint32_t level, uint64_t used) const {
         return cell + (size_t)level * (cap + 1) + used;
@@ -684,8 +690,9 @@ struct KnapsackApp {
                 ok[i] = false;
             }
             if (ok[i]) {
-                gstore16(buf_rsrc(pool + idx), 0,
-                         make_uint4(cl[i], (uint32_t)used[i], value[i], 0u));
+                uint64_t* q = reinterpret_cast<uint64_t*>(pool + idx);
+                u64_store(q, (uint64_t)(uint32_t)used[i] << 32 | cl[i]);
+                u64_store(q + 1, value[i]);
                 child[i] = knap_key(ub[i], cl[i], (uint32_t)idx);
             }
         }
