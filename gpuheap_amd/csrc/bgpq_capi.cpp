@@ -461,6 +461,11 @@ static int insert_calls(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, 
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk insert launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
+    } else if (n <= chunk && solo_pays(h) && bulk_can(h, d_keys, grid, s)) {
+        const hipError_t e = solo_insert(h, d_keys, (int)n, s);
+        if (e != hipSuccess) return fail(BGPQ_EHIP, "insert launch: %s", hipGetErrorString(e));
+        h->bulk_open = true;
+        a.skip = &h->bulk.plan->go;
     }
     h->held += n;
     const hipError_t e = h->row->insert(a, d_keys, n, chunk, resolve_grid(h, grid), s);
@@ -480,6 +485,11 @@ static int delete_calls(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t cal
             bulk_delete(h, d_out, out_keys, calls, ascends, bgpq_default_grid(h->batch_size), s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk delete launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
+        a.skip = &h->bulk.plan->go;
+    } else if (calls == 1 && solo_pays(h) && h->held >= h->batch_size && bulk_can(h, d_out, grid, s)) {
+        const hipError_t e = solo_delete(h, d_out, out_keys, s);
+        if (e != hipSuccess) return fail(BGPQ_EHIP, "delete launch: %s", hipGetErrorString(e));
+        h->bulk_open = true;
         a.skip = &h->bulk.plan->go;
     }
     h->held = std::max<long long>(h->held - pops * h->batch_size, 0);

@@ -66,6 +66,11 @@ bool bulk_one_tile(const bgpq_heap* h, long long keys);
 hipError_t bulk_report(const bgpq_heap* h, int* report, hipStream_t s);
 hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, bool ascends, int cus,
                        hipStream_t s);
+// bgpq_solo.hip: one insertion of `size` keys, one pop; like bulk calls, with
+// plan->go.  solo_pays: the batch sizes where they are the faster ones.
+bool solo_pays(const bgpq_heap* h);
+hipError_t solo_insert(const bgpq_heap* h, const void* keys, int size, hipStream_t s);
+hipError_t solo_delete(const bgpq_heap* h, void* out, long long out_cap, hipStream_t s);
 }  // namespace bgpq
 
 // Records the message returned by bgpq_last_error and returns `code`.
