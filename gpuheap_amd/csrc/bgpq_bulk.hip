@@ -107,7 +107,7 @@ __device__ __forceinline__ void plan_pops(const BulkArgs<K>& a, BulkPlan& pl, lo
         error = ERR_OUTPUT_FULL;
     }
     const long long cut = pops * B + (last ? pbs : 0);
-    const long long tiles = (total + bulk_tile<K>() - 1) / bulk_tile<K>();
+    const long long tiles = (total + a.tile - 1) / a.tile;
     pl.total = (int)total;
     pl.tiles = (int)tiles;
     pl.ascending = ascending;
@@ -362,14 +362,15 @@ __device__ __forceinline__ void count_digits(const unsigned (&cnt)[W][kRadix], u
 //   * 256 threads, one per digit, publish the tile's counts and look back
 //     for those of the tiles before it; meanwhile the keys move into LDS in
 //     digit order, from where each digit's run is written as a whole.
-// What bounds it: vector instructions and LDS accesses (about 80 and 6 for 64
-// keys), at 2^28 u32 keys 850 us a pass, 2.5 TB/s read and written.  It took
-// 1150 us with lane masks built by selects (95 instructions for 64 keys; a
-// mask's step is one v_bitop3 now) and a look-back of one tile at a time,
-// each a round trip of about a microsecond.
-template <typename K>
+// What bounds it: vector instructions (75 for 64 keys, 60% of the time at 2^28
+// u32 keys) and waits for LDS and memory; 800 us a pass there, 2.7 TB/s read
+// and written where a copy reaches 4.6.  It took 1150 us with lane masks built
+// by selects (95 instructions for the ranks alone; a mask's step is one
+// v_bitop3 now) and a look-back of one tile at a time, each a round trip of
+// about a microsecond.
+template <typename K, int T>
 __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, int pass) {
-    constexpr int T = bulk_tile<K>(), U = T / kBulkThreads, W = kBulkThreads / 64;
+    constexpr int U = T / kBulkThreads, W = kBulkThreads / 64;
     constexpr int kWindow = 16;  // tiles looked at together
     __shared__ K keys[T];
     __shared__ unsigned cnt[W][kRadix];
@@ -610,26 +611,30 @@ hipError_t sort_and_finish(const BulkArgs<K>& a, long long keys, hipEvent_t mid,
                            hipStream_t s) {
     constexpr int P = (int)sizeof(K);
     hipLaunchKernelGGL(k_bulk_hist<K>, dim3(blocks_for(keys, 4096, 4 * cus)), dim3(256), 0, s, a);
-    const int grid = blocks_for(keys, bulk_tile<K>(), 3 * cus);
+    constexpr int kSmall = bulk_tile<K>(false), kLarge = bulk_tile<K>(true);
+    const bool large = a.tile == kLarge;
+    const int grid = blocks_for(keys, a.tile, (large ? 2 : 3) * cus);
     for (int p = 0; p < P; ++p) {
         if (p == P - 1 && mid) {
             const hipError_t e = hipEventRecord(mid, s);
             if (e != hipSuccess) return e;
         }
-        hipLaunchKernelGGL(k_bulk_pass<K>, dim3(grid), dim3(kBulkThreads), 0, s, a, p);
+        if (large) hipLaunchKernelGGL((k_bulk_pass<K, kLarge>), dim3(grid), dim3(kBulkThreads), 0, s, a, p);
+        else hipLaunchKernelGGL((k_bulk_pass<K, kSmall>), dim3(grid), dim3(kBulkThreads), 0, s, a, p);
     }
     finish(a, keys, done, cus, s);
     return hipGetLastError();
 }
 
 template <typename K>
-BulkArgs<K> args_for(const bgpq_heap* h) {
+BulkArgs<K> args_for(const bgpq_heap* h, long long keys) {
     BulkArgs<K> a{};
     a.items = (K*)h->items;
     a.ctr = h->ctr;
     a.init_limits = (K)h->init_limits;
     a.batch_num = h->batch_num;
     a.batch_size = h->batch_size;
+    a.tile = bulk_tile<K>(keys >= large_tiles_from<K>());
     a.mem = h->bulk;
     return a;
 }
@@ -637,7 +642,7 @@ BulkArgs<K> args_for(const bgpq_heap* h) {
 template <typename K>
 hipError_t insert_as(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap, long long calls,
                      hipEvent_t mid, int cus, hipStream_t s) {
-    BulkArgs<K> a = args_for<K>(h);
+    BulkArgs<K> a = args_for<K>(h, h->held + n);
     a.keys = (const K*)keys;
     a.n = n;
     a.out = (K*)out;
@@ -659,7 +664,7 @@ hipError_t insert_as(const bgpq_heap* h, const void* keys, long long n, void* ou
 template <typename K>
 hipError_t delete_as(const bgpq_heap* h, void* out, long long out_cap, long long calls, bool ascends, int cus,
                      hipStream_t s) {
-    BulkArgs<K> a = args_for<K>(h);
+    BulkArgs<K> a = args_for<K>(h, h->held);
     a.out = (K*)out;
     a.out_cap = out_cap;
     a.calls = calls;

@@ -27,12 +27,19 @@ constexpr int kRadix = 256;        // 8-bit digits
 constexpr int kMaxPasses = 8;      // of a u64 key
 constexpr int kBulkThreads = 512;  // of a pass's workgroup (8 waves)
 // Keys a workgroup takes at a time (a tile): 32 KB of LDS, which with the
-// counters leaves room for 3 workgroups on a CU.  Smaller tiles are no faster
-// even where these leave CUs idle, since the look-back gets longer (2^20 u32
-// keys: 159, 163, 182 us with 8192, 4096, 2048 keys a tile; u64 rounds of
-// 1.5 M keys in all: 983, 1103, 1415 us with 4096, 2048, 1024).
+// counters leaves room for 3 workgroups on a CU, or 64 KB with room for 2.
+// Large tiles have fewer look-backs and longer runs to write, but a small sort
+// waits longer for its one round of tiles.  From large_tiles_from keys on
+// they are the faster ones (heap sorts, 32 and 64 KB: u64 keys, 1 M 165 and
+// 166 us, 3 M 273 and 238, 30 M 1623 and 1360; u32 keys, 2^25 545 and 563,
+// 2^26 1030 and 1020, 2^28 3849 and 3622).  Smaller tiles than 32 KB are no
+// faster even where they would reach more CUs, since the look-back gets longer
+// (2^20 u32 keys: 159, 163, 182 us with 32, 16, 8 KB; rounds of 1.5 M u64 keys
+// in all: 983, 1103, 1415 us).
 template <typename K>
-constexpr int bulk_tile() { return 32768 / (int)sizeof(K); }
+constexpr int bulk_tile(bool large = false) { return (large ? 65536 : 32768) / (int)sizeof(K); }
+template <typename K>
+constexpr long long large_tiles_from() { return sizeof(K) == 4 ? 1ll << 26 : 1500000; }
 // Above this the lookback words' 30-bit counts would not do.
 constexpr long long kBulkMaxKeys = 1ll << 30;
 
@@ -83,6 +90,7 @@ struct BulkArgs {
     long long n;
     K* out;         // popped, by `calls` deletions
     long long out_cap, calls;
+    int tile;       // keys of a tile
     int from_empty; // only on an empty heap, the output from its start
     int planned;    // the plan is in memory already (k_plan_delete)
     int sorts;      // the sort's kernels follow, not the copy of ascending slots

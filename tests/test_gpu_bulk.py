@@ -234,6 +234,29 @@ def test_bulk_one_tile(gpu, variant, key, order):
         h.close()
 
 
+@pytest.mark.parametrize("key,B,n", [("u64", 1024, 1499999), ("u64", 1024, 1500000), ("u64", 4096, 184 * 8192 - 1),
+                                     ("u64", 256, 184 * 8192), ("u64", 2048, 184 * 8192 + 1), ("u32", 8192, 1 << 26),
+                                     ("u32", 4096, (1 << 26) + 1), ("u32", 8192, (1 << 26) + 16383)])
+@pytest.mark.parametrize("order", ["random", "byte2"])
+def test_bulk_large_tiles(gpu, key, B, n, order):
+    """Counts around the rule for the larger tiles and around whole ones."""
+    print(f"[case] large tiles {key} B={B} n={n} {order}", flush=True)
+    keys = _keys(key, n, n, order)
+    want = np.sort(keys)
+    h = Heap(batch_num_for(n, B), B, key=key)
+    d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer(keys.nbytes)
+    h.heapsort(d, n, d_out=out)
+    assert np.array_equal(out.to_numpy(keys.dtype, n), want)
+    h.insert(d, n)
+    h.set_cursor(0)
+    h.delete(out, n // B // 3)
+    h.delete(out, n // B + 1)
+    G.sync()
+    assert np.array_equal(out.to_numpy(keys.dtype, n), want)
+    assert h.isEmpty() and h.error_flags() == 0
+    h.close()
+
+
 def test_bulk_needs_the_heap_to_itself(gpu):
     """After its view was handed out a heap takes the per-batch kernels only:
     the words of a walked heap differ from the ascending layout."""
