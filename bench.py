@@ -1,9 +1,9 @@
 """Benchmark of the batched GPU priority queue on one MI355X.
 
 One step = one heap sort of N synthetic keys through the heap: insert all
-keys in batch-sized insertion() calls, then deleteRoot/deleteUpdate until the
-heap is empty (the reference harness, test/heap_test.cu:135-162).  The keys
-are generated on the device before timing and stay resident; every step reads
+keys, then pop until the heap is empty (the reference harness,
+test/heap_test.cu:135-162), with Heap.heapsort, which does both as one bulk
+call.  The keys are generated on the device before timing and stay resident; every step reads
 them and writes the sorted output to a second buffer.
 
 Prints one JSON line (the driver's contract) with keys/s, the roofline of the
@@ -35,26 +35,12 @@ HBM_PEAK_GBS = 8000.0
 KEYS = {"u32": (0, np.uint32, 4), "u64": (1, np.uint64, 8)}
 
 
-def levels_sum(m):
-    """S(M) = sum_{k=1..M} floor(log2 k): tree levels below the root summed
-    over the heap sizes 1..M batches."""
-    total, lvl, start = 0, 0, 1
-    while start <= m:
-        end = min(2 * start - 1, m)
-        total += lvl * (end - start + 1)
-        lvl += 1
-        start *= 2
-    return total
-
-
-def alg_bytes(n, b, s):
-    """Algorithmic HBM bytes of a heap sort of n keys, batch b, key size s:
-    insert reads the input once and reads+writes one batch per level; delete
-    writes the output once, reads two children and writes two nodes per level."""
-    m = n // b
-    sm = levels_sum(m)
-    return {"insert": n * s + 2 * b * s * sm, "delete": n * s + 4 * b * s * sm,
-            "total": 2 * n * s + 6 * b * s * sm}
+def alg_bytes(n, s):
+    """HBM bytes of a heap sort of n keys of s bytes, done as one radix sort of
+    s digits (include/bgpq.h, bgpq_heapsort).  Insert phase: the histogram reads
+    the keys and every pass but the last reads and writes them.  Delete phase:
+    the last pass, and the refill of the slots that held them."""
+    return {"insert": n * s * (1 + 2 * (s - 1)), "delete": n * s * 3, "total": n * s * (2 + 2 * s)}
 
 
 def parse_n(v):
@@ -521,7 +507,7 @@ def main():
                         continue
                     r = run_config(args.n, key, variant, b, args.grid_insert, args.grid_delete, 1, 0, order=order,
                                    d_in=d_in, fp_in=fp_in)
-                    ab = alg_bytes(args.n, b, KEYS[key][2])
+                    ab = alg_bytes(args.n, KEYS[key][2])
                     r.update({"n": args.n, "key": key, "order": order, "variant": variant, "batch": b,
                               "hbm_frac_total": ab["total"] / ((r["ms_insert"] + r["ms_delete"]) / 1e3) / 8e12})
                     print(json.dumps(r), flush=True)
@@ -542,15 +528,16 @@ def main():
     if not r["ok"]:
         print("[bench] output check FAILED", file=sys.stderr, flush=True)
     s = KEYS[args.key][2]
-    ab = alg_bytes(args.n, args.batch, s)
+    ab = alg_bytes(args.n, s)
     dom = "delete" if r["ms_delete"] >= r["ms_insert"] else "insert"
     dom_ms = r["ms_" + dom]
     achieved = ab[dom] / (dom_ms / 1e3) / 1e9
     workload = f"heapsort_{args.key}_n{args.n}_{args.variant}_b{args.batch}_{args.order}"
     measured = traffic_for(workload)
-    roofline = {"bound": "hbm", "kernel": f"k_{dom}", "achieved": achieved, "peak": HBM_PEAK_GBS,
+    kernel = f"k_bulk_hist + {s - 1} k_bulk_pass" if dom == "insert" else "k_bulk_pass + k_bulk_finish"
+    roofline = {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-                "traffic": measured.get(f"k_{dom}") if measured else None,
+                "traffic": measured.get(dom) if measured else None,
                 "alg_bytes_per_launch": ab[dom]}
     ok = bool(r["ok"])
     line = {
@@ -583,7 +570,7 @@ def main():
         e = run_config(args.n, args.key, args.variant, b, args.grid_insert, args.grid_delete, 1, 1,
                        order=args.order, d_in=d_in, fp_in=fp_in)
         ok = ok and bool(e["ok"])
-        ab_b = alg_bytes(args.n, b, s)
+        ab_b = alg_bytes(args.n, s)
         extras[str(b)] = {"keys_per_s": e["keys_per_s"], "ms_insert": e["ms_insert"], "ms_delete": e["ms_delete"],
                           "hbm_frac_total": ab_b["total"] / ((e["ms_insert"] + e["ms_delete"]) / 1e3) /
                           (HBM_PEAK_GBS * 1e9), "check": "ok" if e["ok"] else "FAILED"}

@@ -42,6 +42,13 @@ __device__ __forceinline__ int digit_of(K k, int pass) {
     return (int)((k >> (8 * pass)) & (K)(kRadix - 1));
 }
 
+// The same value as one the compiler knows nothing of: what is computed from
+// it is computed anew, not kept in registers from the last use on.
+__device__ __forceinline__ int anew(int x) {
+    asm volatile("" : "+s"(x));
+    return x;
+}
+
 template <typename K>
 __device__ __forceinline__ int ctr_of(const BulkArgs<K>& a, int i) {
     return a.ctr[i * kWordStride];
@@ -305,12 +312,19 @@ __global__ __launch_bounds__(kBulkThreads) void k_bulk_copy(BulkArgs<K> a) {
     }
 }
 
+template <int H>
+__device__ __forceinline__ unsigned rank_of(const unsigned (&rank)[H], int u) {
+    return u % 2 == 0 ? rank[u / 2] & 0xFFFFu : rank[u / 2] >> 16;
+}
 // Ranks of the wave's keys, U rows of 64, among those of the same digit, in
 // order, and the digits' counts in `mine` (zeroed before).  About 80 vector
 // instructions and 3 LDS accesses a row.  A lane finds the lanes with its
 // digit bit by bit: one ballot and one v_bitop3 for each half of the mask.
+// The ranks are kept two to a register: with 32 rows' keys and ranks in
+// registers of their own the large tiles of u32 keys spilled, which wrote 1.7
+// bytes for each byte sorted (790 us a pass at 2^28 keys, 700 so).
 template <typename K, int U>
-__device__ __forceinline__ void rank_rows(const K (&k)[U], int pass, unsigned* mine, unsigned (&rank)[U]) {
+__device__ __forceinline__ void rank_rows(const K (&k)[U], int pass, unsigned* mine, unsigned (&rank)[U / 2]) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int d = digit_of(k[u], pass);
@@ -324,20 +338,23 @@ __device__ __forceinline__ void rank_rows(const K (&k)[U], int pass, unsigned* m
             hi = __builtin_amdgcn_bitop3_b32(hi, (unsigned)(m >> 32), (unsigned)bit, 0x90);
         }
         const unsigned ahead = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
-        rank[u] = ahead | (unsigned)(__popc(lo) + __popc(hi)) << 16;
+        const unsigned both = ahead | (unsigned)(__popc(lo) + __popc(hi)) << 8;
+        rank[u / 2] = u % 2 == 0 ? both : rank[u / 2] | both << 16;
         // one row's masks at a time, and the test for a digit's first lane
         // not before it is needed: 16 rows' masks would spill
-        asm volatile("" : "+v"(rank[u]));
+        asm volatile("" : "+v"(rank[u / 2]));
         __builtin_amdgcn_sched_barrier(0);
     }
+    const int again = anew(pass);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        unsigned* const c = mine + digit_of(k[u], pass);
-        const unsigned before = *c, ahead = rank[u] & 0xFFFFu;
+        unsigned* const c = mine + digit_of(k[u], again);
+        const unsigned before = *c, both = rank_of(rank, u), ahead = both & 0xFFu;
         __builtin_amdgcn_wave_barrier();
-        if (ahead == 0) *c = before + (rank[u] >> 16);
+        if (ahead == 0) *c = before + (both >> 8);
         __builtin_amdgcn_wave_barrier();
-        rank[u] = before + ahead;
+        const unsigned r = before + ahead;  // below 2^16, like both
+        rank[u / 2] = u % 2 == 0 ? (rank[u / 2] & 0xFFFF0000u) | r : (rank[u / 2] & 0xFFFFu) | r << 16;
     }
 }
 
@@ -371,8 +388,8 @@ __device__ __forceinline__ void count_digits(const unsigned (&cnt)[W][kRadix], u
 //   * 256 threads, one per digit, publish the tile's counts and look back
 //     for those of the tiles before it; meanwhile the keys move into LDS in
 //     digit order, from where each digit's run is written as a whole.
-// What bounds it: vector instructions (75 for 64 keys, 60% of the time at 2^28
-// u32 keys) and waits for LDS and memory; 800 us a pass there, 2.7 TB/s read
+// What bounds it: vector instructions (75 for 64 keys, 70% of the time at 2^28
+// u32 keys) and waits for LDS and memory; 700 us a pass there, 3.1 TB/s read
 // and written where a copy reaches 4.6.  It took 1150 us with lane masks built
 // by selects (95 instructions for the ranks alone; a mask's step is one
 // v_bitop3 now) and a look-back of one tile at a time, each a round trip of
@@ -426,7 +443,7 @@ __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, in
 #pragma unroll
             for (int u = 0; u < U; ++u) k[u] = keys[j - j0 + u * 64];  // a thread reads back its own
         }
-        unsigned rank[U];
+        unsigned rank[U / 2];
         unsigned* const mine = cnt[w];
         rank_rows(k, pass, mine, rank);
         __syncthreads();
@@ -444,8 +461,12 @@ __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, in
             for (int i = 0; i < W; ++i) cnt[i][t] = upto + of_wave[i];
         }
         __syncthreads();
+        const int again = anew(pass);
 #pragma unroll
-        for (int u = 0; u < U; ++u) keys[mine[digit_of(k[u], pass)] + rank[u]] = k[u];
+        for (int u = 0; u < U; ++u) {
+            keys[mine[digit_of(k[u], again)] + rank_of(rank, u)] = k[u];
+            if (u % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+        }
         unsigned before = 0;
         if (t < kRadix && tile > 0) {
             const unsigned* const p = look + t;
@@ -478,11 +499,16 @@ __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, in
         if (t < kRadix) to[t] = start + before - upto;  // place of a key = to[digit] + its place in the tile
         __syncthreads();
         if (here == T && !split) {
+            // eight at a time: all of them would take more registers than
+            // the workgroups on a CU leave each other
+#pragma unroll 1
+            for (int u = 0; u < U; u += 8) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int i = u * kBulkThreads + t;
-                const K key = keys[i];
-                dst[to[digit_of(key, pass)] + (unsigned)i] = key;
+                for (int v = 0; v < 8; ++v) {
+                    const int i = (u + v) * kBulkThreads + t;
+                    const K key = keys[i];
+                    dst[to[digit_of(key, pass)] + (unsigned)i] = key;
+                }
             }
         } else {
             for (int i = t; i < here; i += kBulkThreads) {
@@ -564,7 +590,7 @@ __global__ __launch_bounds__(kBulkThreads, 2) void k_bulk_tile(BulkArgs<K> a) {
     for (int u = 0; u < U; ++u) k[u] = keys[j + u * 64];  // a thread reads back its own
 #pragma unroll 1
     for (int pass = 0; pass < P; ++pass) {
-        unsigned rank[U];
+        unsigned rank[U / 2];
 #pragma unroll
         for (int i = 0; i < W * kRadix / kBulkThreads; ++i) (&cnt[0][0])[i * kBulkThreads + t] = 0;
         __syncthreads();
@@ -581,7 +607,7 @@ __global__ __launch_bounds__(kBulkThreads, 2) void k_bulk_tile(BulkArgs<K> a) {
         }
         __syncthreads();
 #pragma unroll
-        for (int u = 0; u < U; ++u) keys[cnt[w][digit_of(k[u], pass)] + rank[u]] = k[u];
+        for (int u = 0; u < U; ++u) keys[cnt[w][digit_of(k[u], pass)] + rank_of(rank, u)] = k[u];
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < U; ++u) k[u] = keys[j + u * 64];
@@ -622,7 +648,10 @@ hipError_t sort_and_finish(const BulkArgs<K>& a, long long keys, hipEvent_t mid,
     hipLaunchKernelGGL(k_bulk_hist<K>, dim3(blocks_for(keys, 4096, 4 * cus)), dim3(256), 0, s, a);
     constexpr int kSmall = bulk_tile<K>(false), kLarge = bulk_tile<K>(true);
     const bool large = a.tile == kLarge;
-    const int grid = blocks_for(keys, a.tile, (large ? 2 : 3) * cus);
+    // two workgroups on a CU, also where three have room: the look-back gets
+    // longer with every tile under way (2^24 u32 keys, 32 KB tiles: 324 us with
+    // two, 353 with three, 363 with one and a half)
+    const int grid = blocks_for(keys, a.tile, 2 * cus);
     for (int p = 0; p < P; ++p) {
         if (p == P - 1 && mid) {
             const hipError_t e = hipEventRecord(mid, s);

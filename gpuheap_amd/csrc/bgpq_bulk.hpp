@@ -26,20 +26,20 @@ namespace bgpq {
 constexpr int kRadix = 256;        // 8-bit digits
 constexpr int kMaxPasses = 8;      // of a u64 key
 constexpr int kBulkThreads = 512;  // of a pass's workgroup (8 waves)
-// Keys a workgroup takes at a time (a tile): 32 KB of LDS, which with the
-// counters leaves room for 3 workgroups on a CU, or 64 KB with room for 2.
-// Large tiles have fewer look-backs and longer runs to write, but a small sort
-// waits longer for its one round of tiles.  From large_tiles_from keys on
-// they are the faster ones (heap sorts, 32 and 64 KB: u64 keys, 1 M 165 and
-// 166 us, 3 M 273 and 238, 30 M 1623 and 1360; u32 keys, 2^25 545 and 563,
-// 2^26 1030 and 1020, 2^28 3849 and 3622).  Smaller tiles than 32 KB are no
+// Keys a workgroup takes at a time (a tile): 32 or 64 KB of LDS, which with the
+// counters leave room for 3 and 2 workgroups on a CU.  Large tiles have fewer
+// look-backs and longer runs to write, but a small sort waits longer for its
+// one round of tiles.  They are the faster ones from large_tiles_from keys on
+// (heap sorts, 32 and 64 KB: u32 keys, 2^20 101 and 113 us, 2^22 172 and 163,
+// 2^24 324 and 301, 2^26 1067 and 918; u64 keys, 300,000 125 and 157, 1 M 161
+// and 163, 1.5 M 196 and 186, 3 M 258 and 238).  Tiles below 32 KB are no
 // faster even where they would reach more CUs, since the look-back gets longer
 // (2^20 u32 keys: 159, 163, 182 us with 32, 16, 8 KB; rounds of 1.5 M u64 keys
 // in all: 983, 1103, 1415 us).
 template <typename K>
 constexpr int bulk_tile(bool large = false) { return (large ? 65536 : 32768) / (int)sizeof(K); }
 template <typename K>
-constexpr long long large_tiles_from() { return sizeof(K) == 4 ? 1ll << 26 : 1500000; }
+constexpr long long large_tiles_from() { return sizeof(K) == 4 ? 1ll << 22 : 1500000; }
 // Above this the lookback words' 30-bit counts would not do.
 constexpr long long kBulkMaxKeys = 1ll << 30;
 

@@ -235,7 +235,8 @@ def test_bulk_one_tile(gpu, variant, key, order):
 
 
 @pytest.mark.parametrize("key,B,n", [("u64", 1024, 1499999), ("u64", 1024, 1500000), ("u64", 4096, 184 * 8192 - 1),
-                                     ("u64", 256, 184 * 8192), ("u64", 2048, 184 * 8192 + 1), ("u32", 8192, 1 << 26),
+                                     ("u64", 256, 184 * 8192), ("u64", 2048, 184 * 8192 + 1), ("u32", 1024, (1 << 22) - 1),
+                                     ("u32", 1024, 1 << 22), ("u32", 512, (1 << 22) + 1), ("u32", 8192, 1 << 26),
                                      ("u32", 4096, (1 << 26) + 1), ("u32", 8192, (1 << 26) + 16383)])
 @pytest.mark.parametrize("order", ["random", "byte2"])
 def test_bulk_large_tiles(gpu, key, B, n, order):
@@ -295,5 +296,49 @@ def test_bulk_calls_on_two_streams(gpu):
     assert hip.hipStreamSynchronize(s) == 0
     assert np.array_equal(out.to_numpy(np.uint32, n), np.sort(keys))
     assert h.isEmpty()
+    h.close()
+    assert hip.hipStreamDestroy(s) == 0
+
+
+@pytest.mark.parametrize("same", [False, True])
+def test_captured_calls_follow_a_bulk_call(gpu, same):
+    """A call that is captured right behind a bulk call, on its stream or on
+    another, is recorded as per-batch kernels; each replay acts on the heap it
+    finds, with eager calls between."""
+    print(f"[case] captured calls same={same}", flush=True)
+    hip = ctypes.CDLL("libamdhip64.so")
+    s, graph, run = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+    B, n = 256, 256 * 4000
+    keys = O.keys_u32(9, n + B)
+    d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer(keys.nbytes)
+    h = Heap(8192, B)
+    a = Heap(64, B)  # loads what a first launch loads
+    a.insert(d, B)
+    a.delete(out, 1)
+    a.view()
+    a.insert(d, B)
+    a.delete(out, 1)
+    a.close()
+    check(lib().bgpq_insert(h._h, d.ptr, n, 0, 0, s if same else None))
+    assert hip.hipStreamBeginCapture(s, 0) == 0
+    check(lib().bgpq_insert(h._h, d.ptr + 4 * n, B, 0, 0, s))
+    check(lib().bgpq_delete(h._h, out.ptr, n, 2, 0, s))
+    assert hip.hipStreamEndCapture(s, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    held, done = np.sort(keys[:n]), 0
+    for i in range(4):
+        assert hip.hipGraphLaunch(run, s) == 0
+        assert hip.hipStreamSynchronize(s) == 0
+        held = np.sort(np.concatenate([held, keys[n:]]))
+        assert np.array_equal(out.to_numpy(np.uint32, done + 2 * B)[done:], held[:2 * B])
+        held, done = held[2 * B:], done + 2 * B
+        h.delete(out, 1, out_keys=n)  # eager
+        G.sync()
+        assert np.array_equal(out.to_numpy(np.uint32, done + B)[done:], held[:B])
+        held, done = held[B:], done + B
+        assert h.checkInsertHeap(), h.last_check_message
+    assert h.itemCount() == len(held) and h.error_flags() == 0
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
     h.close()
     assert hip.hipStreamDestroy(s) == 0
