@@ -124,21 +124,26 @@ static bool capturing(hipStream_t s) {
 }
 
 // The bulk calls end for good once work may run beside them: calls on a second
-// stream, or captured ones, whose graph may run at any time.
+// stream, captured ones, whose graph may run at any time, and kernels of the
+// caller on a view.  The last bulk call is waited for.
+static int end_bulk(bgpq_heap* h) {
+    h->shared = true;
+    if (!h->bulk_open) return BGPQ_OK;
+    // also while this or another thread captures
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = hipEventSynchronize(h->bulk_done);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) return fail(BGPQ_EHIP, "wait for the last bulk call: %s", hipGetErrorString(e));
+    h->bulk_open = false;
+    return BGPQ_OK;
+}
+
 int bgpq_on_stream(bgpq_heap* h, hipStream_t s) {
     std::lock_guard<std::recursive_mutex> hold(h->lock);
-    const bool captured = capturing(s);
-    if (captured || (h->used && s != h->stream)) {
-        h->shared = true;
-        if (h->bulk_open) {
-            // other streams' events may be waited for while this thread captures
-            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-            if (captured) (void)hipThreadExchangeStreamCaptureMode(&mode);
-            const hipError_t e = hipEventSynchronize(h->bulk_done);
-            if (captured) (void)hipThreadExchangeStreamCaptureMode(&mode);
-            if (e != hipSuccess) return fail(BGPQ_EHIP, "wait for the last bulk call: %s", hipGetErrorString(e));
-            h->bulk_open = false;
-        }
+    if ((h->used && s != h->stream) || capturing(s)) {
+        const int rc = end_bulk(h);
+        if (rc) return rc;
     }
     h->used = true;
     h->stream = s;
@@ -293,7 +298,9 @@ int bgpq_reset(bgpq_heap* h, void* stream) {
 
 int bgpq_view(bgpq_heap* h, bgpq_view_t* out) {
     if (!h || !out) return fail(BGPQ_EINVAL, "null argument");
-    h->shared = true;
+    std::lock_guard<std::recursive_mutex> hold(h->lock);
+    const int rc = end_bulk(h);
+    if (rc) return rc;
     out->items = h->items;
     out->status = h->status;
     out->ctr = h->ctr;

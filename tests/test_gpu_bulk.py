@@ -342,3 +342,24 @@ def test_captured_calls_follow_a_bulk_call(gpu, same):
     assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
     h.close()
     assert hip.hipStreamDestroy(s) == 0
+
+
+def test_view_follows_a_bulk_call(gpu):
+    """A heap whose view is handed out right behind a bulk call is complete:
+    a copy on a stream of its own finds the call's counters."""
+    print("[case] view behind a bulk call", flush=True)
+    hip = ctypes.CDLL("libamdhip64.so")
+    s = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+    B, n = 1024, 1 << 26
+    d = DeviceBuffer.from_numpy(O.keys_u32(12, n))
+    h = Heap(batch_num_for(n, B), B)
+    count = ctypes.c_int(-1)
+    G.sync()
+    h.insert(d, n)
+    v = h.view()
+    assert hip.hipMemcpyAsync(ctypes.byref(count), ctypes.c_void_p(v.ctr), ctypes.c_size_t(4), 2, s) == 0
+    assert hip.hipStreamSynchronize(s) == 0
+    assert count.value == n // B
+    h.close()
+    assert hip.hipStreamDestroy(s) == 0
