@@ -100,7 +100,10 @@ __device__ __forceinline__ bool last_to_arrive(int* arrived) {
 template <typename K>
 __device__ __forceinline__ void plan_pops(const BulkArgs<K>& a, BulkPlan& pl, long long nb, int pbs, long long spare,
                                           bool ascending) {
-    const long long B = a.batch_size, total = nb * B + pbs, off = a.from_empty ? 0 : ctr_of(a, CTR_DELETE_COUNT);
+    // a call without pops has nothing to do with the cursor, which the host may
+    // set at any time (bgpq_set_cursor is not ordered on the heap's stream)
+    const long long B = a.batch_size, total = nb * B + pbs;
+    const long long off = a.from_empty || a.calls == 0 ? 0 : ctr_of(a, CTR_DELETE_COUNT);
     long long pops = a.calls < nb ? a.calls : nb;
     const long long room = off <= a.out_cap ? (a.out_cap - off) / B : 0;
     int error = 0;
@@ -526,7 +529,7 @@ template <typename K>
 __device__ __forceinline__ void set_counters(const BulkArgs<K>& a, const BulkPlan& pl) {
     a.ctr[CTR_BATCH_COUNT * kWordStride] = pl.nb_after;
     a.ctr[CTR_PARTIAL * kWordStride] = pl.pbs_after;
-    a.ctr[CTR_DELETE_COUNT * kWordStride] = pl.off + pl.cut;
+    if (a.calls > 0) a.ctr[CTR_DELETE_COUNT * kWordStride] = pl.off + pl.cut;
     a.ctr[CTR_ERROR * kWordStride] |= pl.error;
     if (pl.idle && a.ctr[CTR_BUSY * kWordStride] <= 0) a.ctr[CTR_TERM * kWordStride] = 1;
 }

@@ -363,3 +363,30 @@ def test_view_follows_a_bulk_call(gpu):
     assert count.value == n // B
     h.close()
     assert hip.hipStreamDestroy(s) == 0
+
+
+@pytest.mark.parametrize("key,B,n", [("u32", 1024, 1 << 24), ("u64", 2048, 1 << 22), ("u32", 64, 1 << 12)])
+def test_cursor_set_behind_a_bulk_insertion(gpu, key, B, n):
+    """The output cursor set while a bulk insertion runs on a stream of its own
+    stays: the insertion does not touch it, and the pops start there."""
+    print(f"[case] cursor behind a bulk insertion {key} B={B} n={n}", flush=True)
+    hip = ctypes.CDLL("libamdhip64.so")
+    s = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+    keys = _keys(key, n, 14, "random")
+    h = Heap(2 * batch_num_for(n, B) + 64, B, key=key)
+    d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer(8 * B * keys.itemsize)
+    want = np.sort(keys)
+    check(lib().bgpq_insert(h._h, d.ptr, n, 0, 0, s))
+    check(lib().bgpq_delete(h._h, out.ptr, 8 * B, 5, 0, s))  # leaves the cursor at 5 B
+    assert hip.hipStreamSynchronize(s) == 0
+    assert h.snapshot()[2][2] == 5 * B
+    check(lib().bgpq_insert(h._h, d.ptr, n, 0, 0, s))
+    h.set_cursor(B)
+    check(lib().bgpq_delete(h._h, out.ptr, 8 * B, 2, 0, s))
+    assert hip.hipStreamSynchronize(s) == 0
+    assert h.snapshot()[2][2] == 3 * B and h.error_flags() == 0
+    held = np.sort(np.concatenate([want[5 * B:], want]))
+    assert np.array_equal(out.to_numpy(keys.dtype, 3 * B)[B:], held[:2 * B])
+    h.close()
+    assert hip.hipStreamDestroy(s) == 0
