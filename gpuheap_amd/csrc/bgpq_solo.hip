@@ -169,15 +169,16 @@ struct Solo {
             if (cur == 1) wait_stores();
             __syncthreads();
             const K cmin = X0[0], cmax = X0[B - 1], kmin = X1[0] < X2[0] ? X1[0] : X2[0];
-            if (!(kmin < cmax)) break;  // in order, or no child
-            const bool tr = X1[B - 1] < X2[B - 1];
+            if (!(kmin < cmax) || cl >= last) break;  // in order, or no child (cl < cr)
+            // an absent child is the larger one, also beside keys that are not
+            // below init_limits: the walk never leaves the slots in use
+            const bool tr = cr >= last || X1[B - 1] < X2[B - 1];
             const int tgt = tr ? cr : cl, oth = tr ? cl : cr;
             cl = child(oth, 0);
             cr = child(oth, 1);
             if (cl < last) l.issue(node(a, cl));
             if (cr < last) r.issue(node(a, cr));
             if (tgt < last) wg_merge<K, B, NT>(X1, X2, ToLds<K>{X1}, ToGlobal<K>{node(a, tgt)});
-            // an empty child is the larger one: the other holds the small half
             if (!(cmin < X1[B - 1])) l2g_batch<K, B, NT>(node(a, cur), X1);
             else wg_merge<K, B, NT>(X0, X1, ToGlobal<K>{node(a, cur)}, ToLds<K>{X0});
             __syncthreads();

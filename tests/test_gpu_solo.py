@@ -95,6 +95,36 @@ def test_single_call_limits(gpu, variant):
     h.close()
 
 
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("key,B,cap", [("u32", 64, 9), ("u32", 256, 12), ("u64", 128, 13), ("u32", 4096, 5)])
+@pytest.mark.parametrize("above", [False, True])
+def test_single_pops_stay_in_the_slots(gpu, variant, key, B, cap, above):
+    """Keys at init_limits and above it, which no caller may insert: a pop whose
+    node has a left child only goes down to that one, never to a slot past the
+    last.  Every key comes out, and no free slot is written."""
+    print(f"[case] keys at the limit {variant} {key} B={B} cap={cap} above={above}", flush=True)
+    limit = (1 << 32) - 1 if not above else 1 << 31
+    n = cap * B
+    keys = O.keys_u64(cap, n) >> np.uint64(32) if key == "u64" else O.keys_u32(cap, n)
+    if not above:
+        keys[keys > keys.dtype.type(1 << 31)] = limit
+    h = Heap(cap, B, init_limits=limit, variant=variant, key=key)
+    d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer(keys.nbytes)
+    for i in range(cap):
+        h.insert(d.ptr + i * B * keys.itemsize, B)
+    G.sync()
+    want = np.sort(keys)
+    for i in range(cap):
+        h.delete(out, 1)
+        G.sync()
+        items, status, ctr = h.snapshot()
+        assert (ctr[0], ctr[1], ctr[2], ctr[3]) == (cap - i - 1, 0, (i + 1) * B, 0) and not status.any()
+        assert np.array_equal(np.sort(items[B:B * (cap - i)]), want[(i + 1) * B:])
+        assert (items[B * (cap - i):] == keys.dtype.type(limit)).all()
+    assert np.array_equal(out.to_numpy(keys.dtype, n), want)
+    h.close()
+
+
 def test_single_calls_on_two_streams(gpu):
     """A single call on another stream follows one on the first."""
     hip = ctypes.CDLL("libamdhip64.so")
