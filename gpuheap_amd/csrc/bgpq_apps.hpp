@@ -157,7 +157,7 @@ __device__ void drive(HeapView<uint64_t> h, const App& app, long long* ctl, uint
     K* emit = popped + B;
     int* off = reinterpret_cast<int*>(emit + 4 * B);
     int* aux = off + B + 4;
-    __shared__ int s_n, s_nb, s_part, s_any;
+    __shared__ int s_n, s_nb, s_part, s_any, s_done;
     __shared__ unsigned long long s_scan[NT / 64];
     DevHeap<K, VAR, B, NT> hp{h};
     constexpr bool kThr = App::kThreshold;
@@ -304,15 +304,18 @@ __device__ void drive(HeapView<uint64_t> h, const App& app, long long* ctl, uint
         if (sift) hp.deleteUpdate(kWs);
         if (hp.aborted()) break;
         if (size == 0) {
+            // (a word of its own: with nothing to be had there was no barrier
+            // since s_any was read)
             if (t == 0) {
-                s_any = kThr ? a_load(h.ctr + CTR_TERM * kWordStride) != 0 : ctl_load(ctl, APP_OUTSTANDING) == 0;
-                if (!s_any && ++idle > kMaxIdlePolls) {
+                bool over = kThr ? a_load(h.ctr + CTR_TERM * kWordStride) != 0 : ctl_load(ctl, APP_OUTSTANDING) == 0;
+                if (!over && ++idle > kMaxIdlePolls) {
                     ctl_or(ctl, APP_ERROR, APPERR_IDLE);
-                    s_any = 1;
+                    over = true;
                 }
+                s_done = over;
             }
             __syncthreads();
-            const bool done = s_any != 0;
+            const bool done = s_done != 0;
             __syncthreads();
             if (done) break;
             backoff();

@@ -70,3 +70,24 @@ def test_children_and_partial_keys_over_two_batches(gpu, team):
         res, _ = S.batch_run(qs, budget)
         for r, a, b in zip(res, got, want):
             assert r["status"] == 0 and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("variant", ["buitdd", "tditdd"])
+@pytest.mark.parametrize("B", [256, 2048])
+def test_idle_workgroups_leave_together(gpu, variant, B):
+    """Searches with one key at a time by 120 workgroups: most of them find
+    nothing from their first pass to the last, and all waves of each must take
+    the same way when the search ends."""
+    print(f"[case] idle workgroups {variant} B={B}", flush=True)
+    n = 40  # a path
+    g = A.Graph(np.minimum(np.arange(n + 1), n - 1).astype(np.int32), np.arange(1, n, dtype=np.int32),
+                np.full(n - 1, 3, np.uint32))
+    free = np.ones(2 * 24, np.uint8)
+    w, v, cap = A.knapsack_instance(12, 1)
+    best, (cost, _) = O.knapsack_dp(w, v, cap), O.astar(free, 24, 2)
+    with _heap(B, 1 << 14, variant) as h:
+        for _ in range(10):
+            dist, _ = A.sssp(h, g, source=0, grid=120)
+            assert np.array_equal(dist, 3 * np.arange(n)) and h.isEmpty()
+            assert A.astar(h, A.GridMap(free, 24, 2), grid=120)[0] == cost
+            assert A.knapsack(h, w, v, cap, grid=120)[0] == best
