@@ -134,7 +134,13 @@ __device__ __forceinline__ void plan_pops(const BulkArgs<K>& a, BulkPlan& pl, lo
     pl.fill_lo = (nb - pops + 1) * B;
     pl.fill_hi = spare + through;
     pl.error = error;
-    pl.idle = a.calls > pops + (last ? 1 : 0) && total == cut;
+    // The vote as the workgroups of a per-batch call would leave it, each with
+    // every `poppers`th call, the calls in order: a workgroup is busy from its
+    // first pop until a call of its finds nothing, and those calls come last.
+    const long long none = a.calls - pops - (last ? 1 : 0);
+    const long long workgroups = a.calls < a.poppers ? a.calls : a.poppers;
+    pl.idle = none > 0;
+    pl.busy = (int)(workgroups - (none < workgroups ? none : workgroups));
     pl.go = total > 0 && total < kBulkMaxKeys && tiles <= a.mem.tiles_max &&
             spare + through <= ((long long)a.batch_num + 1) * B && (cut == 0 || off + total < (1ll << 31)) &&
             ctr_of(a, CTR_ABORT) == 0;
@@ -531,7 +537,9 @@ __device__ __forceinline__ void set_counters(const BulkArgs<K>& a, const BulkPla
     a.ctr[CTR_PARTIAL * kWordStride] = pl.pbs_after;
     if (a.calls > 0) a.ctr[CTR_DELETE_COUNT * kWordStride] = pl.off + pl.cut;
     a.ctr[CTR_ERROR * kWordStride] |= pl.error;
-    if (pl.idle && a.ctr[CTR_BUSY * kWordStride] <= 0) a.ctr[CTR_TERM * kWordStride] = 1;
+    const int busy = a.ctr[CTR_BUSY * kWordStride] + pl.busy;
+    a.ctr[CTR_BUSY * kWordStride] = busy;
+    if (pl.idle && busy <= 0) a.ctr[CTR_TERM * kWordStride] = 1;
 }
 
 // Batches that stay come back from the spare slots (ascending slots only);
@@ -682,13 +690,14 @@ BulkArgs<K> args_for(const bgpq_heap* h, long long keys) {
 
 template <typename K>
 hipError_t insert_as(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap, long long calls,
-                     hipEvent_t mid, int cus, hipStream_t s) {
+                     int poppers, hipEvent_t mid, int cus, hipStream_t s) {
     BulkArgs<K> a = args_for<K>(h, h->held + n);
     a.keys = (const K*)keys;
     a.n = n;
     a.out = (K*)out;
     a.out_cap = out_cap;
     a.calls = calls;
+    a.poppers = poppers;
     a.from_empty = mid != nullptr;
     clear_last_error();
     if (bulk_one_tile(h, h->held + n)) {
@@ -703,12 +712,13 @@ hipError_t insert_as(const bgpq_heap* h, const void* keys, long long n, void* ou
 }
 
 template <typename K>
-hipError_t delete_as(const bgpq_heap* h, void* out, long long out_cap, long long calls, bool ascends, int cus,
-                     hipStream_t s) {
+hipError_t delete_as(const bgpq_heap* h, void* out, long long out_cap, long long calls, int poppers, bool ascends,
+                     int cus, hipStream_t s) {
     BulkArgs<K> a = args_for<K>(h, h->held);
     a.out = (K*)out;
     a.out_cap = out_cap;
     a.calls = calls;
+    a.poppers = poppers;
     a.planned = 1;
     a.sorts = !ascends;
     clear_last_error();
@@ -723,9 +733,9 @@ hipError_t delete_as(const bgpq_heap* h, void* out, long long out_cap, long long
 }  // namespace
 
 hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap,
-                       long long calls, hipEvent_t mid, int cus, hipStream_t s) {
-    return h->key_type == BGPQ_KEY_U64 ? insert_as<uint64_t>(h, keys, n, out, out_cap, calls, mid, cus, s)
-                                       : insert_as<uint32_t>(h, keys, n, out, out_cap, calls, mid, cus, s);
+                       long long calls, int poppers, hipEvent_t mid, int cus, hipStream_t s) {
+    return h->key_type == BGPQ_KEY_U64 ? insert_as<uint64_t>(h, keys, n, out, out_cap, calls, poppers, mid, cus, s)
+                                       : insert_as<uint32_t>(h, keys, n, out, out_cap, calls, poppers, mid, cus, s);
 }
 bool bulk_one_tile(const bgpq_heap* h, long long keys) {
     return keys <= (h->key_type == BGPQ_KEY_U64 ? bulk_tile<uint64_t>() : bulk_tile<uint32_t>());
@@ -734,10 +744,10 @@ hipError_t bulk_report(const bgpq_heap* h, int* report, hipStream_t s) {
     hipLaunchKernelGGL(k_bulk_report, dim3(1), dim3(64), 0, s, h->bulk.plan, h->ctr, report);
     return hipGetLastError();
 }
-hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, bool ascends, int cus,
-                       hipStream_t s) {
-    return h->key_type == BGPQ_KEY_U64 ? delete_as<uint64_t>(h, out, out_cap, calls, ascends, cus, s)
-                                       : delete_as<uint32_t>(h, out, out_cap, calls, ascends, cus, s);
+hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, int poppers, bool ascends,
+                       int cus, hipStream_t s) {
+    return h->key_type == BGPQ_KEY_U64 ? delete_as<uint64_t>(h, out, out_cap, calls, poppers, ascends, cus, s)
+                                       : delete_as<uint32_t>(h, out, out_cap, calls, poppers, ascends, cus, s);
 }
 
 }  // namespace bgpq

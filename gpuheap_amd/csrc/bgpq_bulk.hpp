@@ -43,7 +43,7 @@ constexpr long long large_tiles_from() { return sizeof(K) == 4 ? 1ll << 22 : 150
 // Above this the lookback words' 30-bit counts would not do.
 constexpr long long kBulkMaxKeys = 1ll << 30;
 
-// What a bulk call does, decided by k_plan_insert / k_plan_delete.
+// What a bulk call does, decided by plan_insert or k_plan_delete.
 struct BulkPlan {
     int go;               // 0: the per-batch kernel runs instead
     int ascending;        // delete: the slots already ascend, no sort needed
@@ -58,7 +58,8 @@ struct BulkPlan {
     long long spare;      // first key index of the free slots used
     long long fill_lo, fill_hi;  // key range refilled with init_limits
     int error;            // error flags to raise
-    int idle;             // a deletion found nothing (termination vote)
+    // termination vote: deletions that found nothing, and workgroups left busy
+    int idle, busy;
     int active;           // passes that move keys
     int order[kMaxPasses];  // position of a pass among them, -1: skipped
     int through_out;        // the passes alternate between the free slots and the output
@@ -90,6 +91,7 @@ struct BulkArgs {
     long long n;
     K* out;         // popped, by `calls` deletions
     long long out_cap, calls;
+    int poppers;    // workgroups that would pop them one after the other (the vote counts them)
     int tile;       // keys of a tile
     int from_empty; // only on an empty heap, the output from its start
     int planned;    // the plan is in memory already (k_plan_delete)

@@ -464,7 +464,7 @@ static int insert_calls(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, 
     if (rc) return rc;
     HeapArgs a = args_of(h);
     if (insert_pays(h, (n + chunk - 1) / chunk, h->held + n) && bulk_can(h, d_keys, grid, s)) {
-        const hipError_t e = bulk_insert(h, d_keys, n, nullptr, 0, 0, nullptr, bgpq_default_grid(h->batch_size), s);
+        const hipError_t e = bulk_insert(h, d_keys, n, nullptr, 0, 0, 0, nullptr, bgpq_default_grid(h->batch_size), s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk insert launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
@@ -488,8 +488,8 @@ static int delete_calls(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t cal
     HeapArgs a = args_of(h, out_keys);
     const long long pops = std::min<long long>(calls, (h->held + h->batch_size - 1) / h->batch_size);
     if (delete_pays(h, pops, h->held, ascends) && bulk_can(h, d_out, grid, s)) {
-        const hipError_t e =
-            bulk_delete(h, d_out, out_keys, calls, ascends, bgpq_default_grid(h->batch_size), s);
+        const hipError_t e = bulk_delete(h, d_out, out_keys, calls, resolve_grid(h, grid), ascends,
+                                         bgpq_default_grid(h->batch_size), s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk delete launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
@@ -548,8 +548,8 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
     const long long in = (n_insert + chunk - 1) / chunk, all = h->held + n_insert;
     const long long pops = std::min<long long>(calls, (all + h->batch_size - 1) / h->batch_size);
     if (sort_pays(h, in, pops, all) && bulk_can(h, d_keys, grid, s) && bulk_can(h, d_out, grid, s)) {
-        const hipError_t e =
-            bulk_insert(h, d_keys, n_insert, d_out, out_keys, calls, nullptr, bgpq_default_grid(h->batch_size), s);
+        const hipError_t e = bulk_insert(h, d_keys, n_insert, d_out, out_keys, calls, grid - grid / 2, nullptr,
+                                         bgpq_default_grid(h->batch_size), s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
@@ -566,11 +566,12 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
 // goes on as if the call had not been made.  Nothing is asked of the device
 // before or between (of 150 us for 2^20 u32 keys, 60 were two copies of the
 // counters, a memset and the making of events).
-static int bulk_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n, int64_t pops, float* ms_insert,
-                         float* ms_delete, hipStream_t s, bool* done) {
+static int bulk_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n, int64_t pops, int poppers,
+                         float* ms_insert, float* ms_delete, hipStream_t s, bool* done) {
     hipEvent_t* const ev = h->sort_events;
     HIPCHK(hipEventRecord(ev[0], s));
-    const hipError_t e = bulk_insert(h, d_in, n, d_out, n, pops + 1, ev[1], bgpq_default_grid(h->batch_size), s);
+    const hipError_t e = bulk_insert(h, d_in, n, d_out, n, pops + 1, poppers, ev[1],
+                                     bgpq_default_grid(h->batch_size), s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk launch: %s", hipGetErrorString(e));
     h->bulk_open = h->ascends = true;
     HIPCHK(hipEventRecord(ev[2], s));
@@ -609,7 +610,7 @@ int bgpq_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n, int ch
         bulk_can(h, d_in, grid_insert, s) && bulk_can(h, d_out, grid_delete, s)) {
         if (!h->sort_report) HIPCHK(hipHostMalloc((void**)&h->sort_report, kReportWords * sizeof(int), 0));
         bool done = false;
-        rc = bulk_heapsort(h, d_in, d_out, n, pops, ms_insert, ms_delete, s, &done);
+        rc = bulk_heapsort(h, d_in, d_out, n, pops, resolve_grid(h, grid_delete), ms_insert, ms_delete, s, &done);
         if (rc || done) return rc;
     }
     int c[CTR_WORDS];

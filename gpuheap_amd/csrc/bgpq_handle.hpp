@@ -52,7 +52,8 @@ int bgpq_on_stream(bgpq_heap* h, hipStream_t s);
 namespace bgpq {
 // The launch sequences of bgpq_bulk.hip.  A per-batch kernel with
 // HeapArgs::skip = &plan->go must follow them, unless the plan cannot refuse.
-// bulk_insert: n keys in, then `calls` deletions (0 for none).  With `mid` a
+// bulk_insert: n keys in, then `calls` deletions (0 for none), which count in
+// the termination vote as those of `poppers` workgroups.  With `mid` a
 // heap sort: refused unless the heap is empty, the output starts at its first
 // key whatever the cursor, and `mid` is recorded before the pass of the
 // highest digit.
@@ -60,12 +61,12 @@ namespace bgpq {
 // bulk_delete: `ascends` where the slots are expected to ascend (a plan that
 // finds otherwise refuses).
 hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, void* out, long long out_cap,
-                       long long calls, hipEvent_t mid, int cus, hipStream_t s);
+                       long long calls, int poppers, hipEvent_t mid, int cus, hipStream_t s);
 // Whether an insertion that makes `keys` keys in all is sorted by one workgroup.
 bool bulk_one_tile(const bgpq_heap* h, long long keys);
 hipError_t bulk_report(const bgpq_heap* h, int* report, hipStream_t s);
-hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, bool ascends, int cus,
-                       hipStream_t s);
+hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, int poppers, bool ascends,
+                       int cus, hipStream_t s);
 // bgpq_solo.hip: one insertion of `size` keys, one pop; like bulk calls, with
 // plan->go.  solo_pays: the batch sizes where they are the faster ones.
 bool solo_pays(const bgpq_heap* h);

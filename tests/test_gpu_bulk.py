@@ -390,3 +390,38 @@ def test_cursor_set_behind_a_bulk_insertion(gpu, key, B, n):
     assert np.array_equal(out.to_numpy(keys.dtype, 3 * B)[B:], held[:2 * B])
     h.close()
     assert hip.hipStreamDestroy(s) == 0
+
+
+@pytest.mark.parametrize("variant", VARIANTS)
+@pytest.mark.parametrize("B,batches,grid", [(64, 300, 32), (256, 100, 256), (1024, 40, 7)])
+def test_bulk_pops_vote(gpu, variant, B, batches, grid):
+    """Bulk pops take part in the termination vote as the per-batch kernels'
+    workgroups do (counters 5 and 6: busy workgroups, the vote's end): on a
+    heap whose view was handed out, and by the rule where only one answer is
+    possible.  Not ended while workgroups are busy, ended once each of them has
+    found nothing."""
+    n = B * batches + (B // 2 if variant in PB else 0)
+    got = -(-n // B)
+    keys = O.keys_u32(batches, n)
+    d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer(keys.nbytes)
+    for calls, busy, end in ((batches - 1, min(grid, batches - 1), 0), (got, min(grid, got), 0),
+                             (got + 1, min(grid, got + 1) - 1, 0), (got + 8 * grid, 0, 1)):
+        print(f"[case] vote {variant} B={B} batches={batches} grid={grid} calls={calls}", flush=True)
+        for how in ("shared", "pops", "concurrent", "heapsort"):
+            if how == "heapsort" and calls != got + 1:
+                continue
+            h = Heap(batch_num_for(n, B) + 64, B, variant=variant)
+            if how == "shared":
+                h.view()
+            if how == "heapsort":
+                h.heapsort(d, n, grid_delete=grid, d_out=out)
+            elif how == "concurrent":
+                h.concurrent(d, n, out, calls, grid=2 * grid, out_keys=n)
+            else:
+                h.insert(d, n)
+                h.delete(out, calls, grid=grid, out_keys=n)
+            G.sync()
+            ctr = h.snapshot()[2]
+            assert (ctr[5], ctr[6]) == (busy, end), how
+            assert h.ifTerminate() == bool(end) and ctr[2] == min(calls * B, n)
+            h.close()
