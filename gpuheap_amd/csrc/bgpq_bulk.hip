@@ -5,7 +5,7 @@
 //   k_plan_delete                   pops only: what to do (BulkPlan)
 //   k_bulk_hist                     key counts of every digit of every pass
 //                                   (and the plan, where there are insertions)
-//   k_bulk_pass, once per digit     one pass of a least-digit-first radix sort
+//   k_bulk_pass, a launch a digit   one pass of a least-digit-first radix sort
 //   k_bulk_finish                   free slots refilled, counters set
 // or, for insertions that make no more than a tile of keys in all, with pops or
 // without, k_bulk_tile alone.
@@ -285,7 +285,8 @@ __global__ __launch_bounds__(256) void k_bulk_hist(BulkArgs<K> a) {
             }
         }
         int at = 0;
-        for (int p = 0; p < P; ++p) pl.order[p] = moves[p] ? at++ : -1;
+        for (int p = 0; p < P; ++p)
+            if (moves[p]) pl.digit[at++] = p;
         pl.active = n;
         // where all keys leave, the output is the second buffer, so that the
         // slots in use need no refill twice as long as the keys
@@ -404,7 +405,7 @@ __device__ __forceinline__ void count_digits(const unsigned (&cnt)[W][kRadix], u
 // v_bitop3 now) and a look-back of one tile at a time, each a round trip of
 // about a microsecond.
 template <typename K, int T>
-__global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, int pass) {
+__global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, int launch) {
     constexpr int U = T / kBulkThreads, W = kBulkThreads / 64;
     constexpr int kWindow = 16;  // tiles looked at together
     __shared__ K keys[T];
@@ -414,8 +415,10 @@ __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, in
     __shared__ int s_tile;
     const BulkPlan& pl = *a.mem.plan;
     if (!pl.go || pl.ascending) return;
-    const int ord = pl.order[pass];
+    // dropped passes are the first launches: the last one always hands the keys out
+    const int ord = launch - ((int)sizeof(K) - pl.active);
     if (ord < 0) return;
+    const int pass = __builtin_amdgcn_readfirstlane(pl.digit[ord]);
     const bool first = ord == 0, last = ord == pl.active - 1;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int total = pl.total, tiles = pl.tiles;
@@ -650,8 +653,8 @@ void finish(const BulkArgs<K>& a, long long keys, hipEvent_t done, int cus, hipS
                           a);
 }
 
-// The sort of about `keys` keys; `mid`, if any, is recorded before the pass of
-// the highest digit.
+// The sort of about `keys` keys; `mid`, if any, is recorded before the last
+// pass, which hands the keys out.
 template <typename K>
 hipError_t sort_and_finish(const BulkArgs<K>& a, long long keys, hipEvent_t mid, hipEvent_t done, int cus,
                            hipStream_t s) {

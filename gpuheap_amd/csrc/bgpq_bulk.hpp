@@ -60,8 +60,8 @@ struct BulkPlan {
     int error;            // error flags to raise
     // termination vote: deletions that found nothing, and workgroups left busy
     int idle, busy;
-    int active;           // passes that move keys
-    int order[kMaxPasses];  // position of a pass among them, -1: skipped
+    int active;           // passes that move keys: the last launches
+    int digit[kMaxPasses];  // the digit of each of them
     int through_out;        // the passes alternate between the free slots and the output
 };
 

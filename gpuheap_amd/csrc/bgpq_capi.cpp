@@ -560,12 +560,12 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
     return BGPQ_OK;
 }
 
-// A heap sort as one bulk call: both halves are one sort, and the pass of the
-// highest digit, which hands the keys out, counts as the second.  *done is
-// false where the heap turned out not to be empty or is aborted: the caller
-// goes on as if the call had not been made.  Nothing is asked of the device
-// before or between (of 150 us for 2^20 u32 keys, 60 were two copies of the
-// counters, a memset and the making of events).
+// A heap sort as one bulk call: both halves are one sort, and its last pass,
+// which hands the keys out, counts as the second.  *done is false where the heap
+// turned out not to be empty or is aborted: the caller goes on as if the call
+// had not been made.  Nothing is asked of the device before or between (of 150
+// us for 2^20 u32 keys, 60 were two copies of the counters, a memset and the
+// making of events).
 static int bulk_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n, int64_t pops, int poppers,
                          float* ms_insert, float* ms_delete, hipStream_t s, bool* done) {
     hipEvent_t* const ev = h->sort_events;

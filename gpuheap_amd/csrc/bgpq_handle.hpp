@@ -55,8 +55,8 @@ namespace bgpq {
 // bulk_insert: n keys in, then `calls` deletions (0 for none), which count in
 // the termination vote as those of `poppers` workgroups.  With `mid` a
 // heap sort: refused unless the heap is empty, the output starts at its first
-// key whatever the cursor, and `mid` is recorded before the pass of the
-// highest digit.
+// key whatever the cursor, and `mid` is recorded before the pass that hands
+// the keys out (before the one kernel of a sort of one tile).
 // bulk_report: kReportWords words of pinned memory, behind a heap sort.
 // bulk_delete: `ascends` where the slots are expected to ascend (a plan that
 // finds otherwise refuses).

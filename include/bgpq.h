@@ -85,7 +85,8 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
  * 2*ceil(n/batch_size) slots.  Optional outputs: the insert and delete phase
  * times in ms, from HIP events on `stream`.  Where the heap has itself to itself
  * and the calls are many, both phases are one sort: the delete phase is then
- * its last pass, which hands the keys out, and what follows. */
+ * its last pass, which hands the keys out, and what follows (all of a sort that
+ * one workgroup does, of at most 8192 u32 or 4096 u64 keys). */
 int bgpq_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n, int chunk, int grid_insert,
                   int grid_delete, float* ms_insert, float* ms_delete, void* stream);
 

@@ -425,3 +425,26 @@ def test_bulk_pops_vote(gpu, variant, B, batches, grid):
             assert (ctr[5], ctr[6]) == (busy, end), how
             assert h.ifTerminate() == bool(end) and ctr[2] == min(calls * B, n)
             h.close()
+
+
+@pytest.mark.parametrize("key,n,bits", [("u32", 1 << 26, 24), ("u32", 1 << 26, 9), ("u64", 1 << 24, 40)])
+def test_delete_phase_hands_the_keys_out(gpu, key, n, bits):
+    """A heap sort's delete phase holds the pass that hands the keys out also
+    where the highest digits are the same for all keys and their passes are
+    dropped.  That pass moves as many bytes as with all passes, so the phase
+    takes about as long; without it, it would be the refill alone, a quarter."""
+    print(f"[case] delete phase {key} n={n} bits={bits}", flush=True)
+    B = 1024
+    keys = _keys(key, n, 15, "random")
+    few = keys >> keys.dtype.type(keys.itemsize * 8 - bits)
+    h = Heap(batch_num_for(n, B), B, key=key)
+    out = DeviceBuffer(keys.nbytes)
+    ms = []
+    for k in (keys, few):
+        d = DeviceBuffer.from_numpy(k)
+        ms.append(np.median([h.heapsort(d, n, d_out=out) for _ in range(7)], axis=0)[1])
+        assert np.array_equal(out.to_numpy(k.dtype, n), np.sort(k))
+        d.free()
+    print(f"[case] delete phase {ms[0]:.3f} ms, {bits}-bit keys {ms[1]:.3f} ms", flush=True)
+    assert ms[1] > 0.5 * ms[0]
+    h.close()
