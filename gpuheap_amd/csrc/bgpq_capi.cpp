@@ -616,7 +616,8 @@ int bgpq_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n, int ch
     int c[CTR_WORDS];
     rc = counters(h, c);
     if (rc) return rc;
-    if (h->held != 0) return fail(BGPQ_EINVAL, "heap sort needs an empty heap (%lld items)", h->held);
+    const long long items = (long long)c[CTR_BATCH_COUNT] * B + c[CTR_PARTIAL];
+    if (items != 0) return fail(BGPQ_EINVAL, "heap sort needs an empty heap (%lld items)", items);
     if (!fits)
         return fail(BGPQ_EINVAL, "capacity: %lld keys need batch_num >= %lld", (long long)n,
                     (long long)(2 * ((n + B - 1) / B)));

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <mutex>
 
 #include "bgpq.h"
@@ -24,8 +25,9 @@ struct bgpq_heap {
     bgpq::BulkMem bulk;  // working words of the bulk calls, behind ctr and items
     // Keys the heap holds as far as the host can tell without asking the
     // device.  It only chooses between the per-batch and the bulk kernels;
-    // those act on the counters they find.
-    long long held;
+    // those act on the counters they find.  Atomic: whoever reads the counters
+    // (bgpq_item_count and the like) corrects it beside other threads' calls.
+    std::atomic<long long> held;
     // The bulk kernels need the heap to themselves.  They stay off once the
     // view was handed out (kernels of the caller may use the heap at any
     // time) or calls came on more than one stream.

@@ -1,0 +1,126 @@
+// The C ABI's host code on a stand-in for the HIP runtime and the kernels:
+// device memory is host memory, a launch only leaves a note.  It shows what the
+// host decides where no GPU can (a device short of memory) or need (two threads).
+//   capi_host counters   two threads: calls on a heap, and reads of its counters
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <thread>
+
+#include "bgpq_handle.hpp"
+
+using namespace bgpq;
+
+// ------------------------------------------------------------- HIP runtime
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) {
+    *p = calloc(1, n);
+    return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipFree(void* p) {
+    free(p);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostFree(void* p) { return hipFree(p); }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
+    memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) {
+    return hipMemcpy(d, s, n, k);
+}
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) {
+    memset(d, v, n);
+    return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) { return memset(p, 0, sizeof *p), hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "stand-in"; }
+hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = (hipEvent_t)1, hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* t, hipEvent_t, hipEvent_t) { return *t = 0, hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
+    return *s = hipStreamCaptureStatusNone, hipSuccess;
+}
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
+}
+
+// ----------------------------------------------------------------- kernels
+namespace bgpq {
+static hipError_t row_insert(const HeapArgs&, const void*, long long, int, int, hipStream_t) { return hipSuccess; }
+static hipError_t row_del(const HeapArgs&, void*, long long, int, hipStream_t) { return hipSuccess; }
+static hipError_t row_conc(const HeapArgs&, const void*, long long, int, void*, long long, int, hipStream_t) {
+    return hipSuccess;
+}
+static const LaunchRow* rows() {
+    static LaunchRow r[kNumBatchSizes];
+    static const bool made = [] {
+        for (int i = 0; i < kNumBatchSizes; ++i) r[i] = LaunchRow{64 << i, nullptr, nullptr, row_insert, row_del, row_conc};
+        return true;
+    }();
+    (void)made;
+    return r;
+}
+const LaunchRow* rows_u32_v0() { return rows(); }
+const LaunchRow* rows_u32_v1() { return rows(); }
+const LaunchRow* rows_u32_v2() { return rows(); }
+const LaunchRow* rows_u32_v3() { return rows(); }
+const LaunchRow* rows_u64_v0() { return rows(); }
+const LaunchRow* rows_u64_v1() { return rows(); }
+const LaunchRow* rows_u64_v2() { return rows(); }
+const LaunchRow* rows_u64_v3() { return rows(); }
+hipError_t fill_u32(void*, long long, uint32_t, hipStream_t) { return hipSuccess; }
+hipError_t fill_u64(void*, long long, uint64_t, hipStream_t) { return hipSuccess; }
+hipError_t clear_u32(void*, int*, int*, int, int, uint32_t, hipStream_t) { return hipSuccess; }
+hipError_t clear_u64(void*, int*, int*, int, int, uint64_t, hipStream_t) { return hipSuccess; }
+hipError_t bulk_insert(const bgpq_heap*, const void*, long long, void*, long long, long long, int, hipEvent_t, int,
+                       hipStream_t) {
+    return hipSuccess;
+}
+hipError_t bulk_delete(const bgpq_heap*, void*, long long, long long, int, bool, int, hipStream_t) {
+    return hipSuccess;
+}
+hipError_t bulk_report(const bgpq_heap*, int*, hipStream_t) { return hipSuccess; }
+bool bulk_one_tile(const bgpq_heap*, long long) { return false; }
+bool solo_pays(const bgpq_heap*) { return true; }
+hipError_t solo_insert(const bgpq_heap*, const void*, int, hipStream_t) { return hipSuccess; }
+hipError_t solo_delete(const bgpq_heap*, void*, long long, hipStream_t) { return hipSuccess; }
+}  // namespace bgpq
+
+#define CHECK(x)                                                                     \
+    do {                                                                             \
+        if (!(x)) return printf("%s:%d: %s\n", __FILE__, __LINE__, #x), 1;           \
+    } while (0)
+
+static int counters() {
+    bgpq_heap* h = nullptr;
+    CHECK(bgpq_create(&h, BGPQ_BUITDD, BGPQ_KEY_U32, 64, 64, 0xFFFFFFFFu) == BGPQ_OK);
+    uint32_t keys[64] = {}, out[64];
+    std::thread reader([&] {
+        int64_t n = 0;
+        for (int i = 0; i < 2000; ++i) bgpq_item_count(h, &n);
+    });
+    int rc = BGPQ_OK;
+    for (int i = 0; i < 2000 && rc == BGPQ_OK; ++i) {
+        rc = bgpq_insert(h, keys, 64, 0, 0, nullptr);
+        if (rc == BGPQ_OK) rc = bgpq_delete(h, out, 64, 1, 0, nullptr);
+    }
+    reader.join();
+    CHECK(rc == BGPQ_OK);
+    bgpq_destroy(h);
+    return 0;
+}
+
+int main(int argc, char** argv) {
+    const char* what = argc > 1 ? argv[1] : "";
+    if (!strcmp(what, "counters")) return counters();
+    return 2;
+}
