@@ -87,7 +87,7 @@ static size_t bulk_fixed_bytes() {
     return up256(ctr_bytes()) + up256(sizeof(BulkPlan)) + up256(sizeof(unsigned) * kSortWords);
 }
 static size_t bulk_look_bytes(const bgpq_heap* h) { return sizeof(unsigned) * kRadix * (size_t)bulk_tiles_max(h); }
-static void set_bulk_mem(bgpq_heap* h) {
+static void set_bulk_mem(bgpq_heap* h, bool look) {
     char* p = (char*)h->ctr + up256(ctr_bytes());
     h->bulk.plan = (BulkPlan*)p;
     p += up256(sizeof(BulkPlan));
@@ -97,7 +97,7 @@ static void set_bulk_mem(bgpq_heap* h) {
     p = (char*)h->items + up256(items_bytes(h));
     h->bulk.look[0] = (unsigned*)p;
     h->bulk.look[1] = (unsigned*)(p + bulk_look_bytes(h));
-    h->bulk.tiles_max = bulk_tiles_max(h);
+    h->bulk.tiles_max = look ? bulk_tiles_max(h) : 0;
 }
 
 static int fill_items(bgpq_heap* h, hipStream_t s) {
@@ -254,16 +254,29 @@ int bgpq_create(bgpq_heap** out, int variant, int key_type, int batch_num, int b
     h->batch_size = batch_size;
     h->init_limits = init_limits;
     h->row = &rows_for(key_type, variant)[bi];
-    const size_t bytes = up256(items_bytes(h)) + 2 * bulk_look_bytes(h);
-    auto alloc = [](void** p, size_t n) { return hipMalloc(p, n); };
-    hipError_t e = alloc(&h->items, bytes);
-    if (e == hipSuccess) e = alloc((void**)&h->status, status_bytes(batch_num));
-    if (e == hipSuccess) e = alloc((void**)&h->ctr, bulk_fixed_bytes());
+    // A device that has no room for the lookback words (up to half a gigabyte)
+    // beside the slots: the heap goes without them and without bulk calls.
+    size_t bytes = 0;
+    hipError_t e = hipSuccess;
+    for (const bool bulk : {true, false}) {
+        bytes = items_bytes(h);
+        if (bulk) bytes = up256(bytes) + 2 * bulk_look_bytes(h);
+        e = hipMalloc(&h->items, bytes);
+        if (e == hipSuccess) e = hipMalloc((void**)&h->status, status_bytes(batch_num));
+        if (e == hipSuccess) e = hipMalloc((void**)&h->ctr, bulk_fixed_bytes());
+        if (e == hipSuccess) {
+            set_bulk_mem(h, bulk);
+            break;
+        }
+        if (h->items) (void)hipFree(h->items);
+        if (h->status) (void)hipFree(h->status);
+        h->items = nullptr;
+        h->status = nullptr;
+    }
     if (e != hipSuccess) {
         bgpq_destroy(h);
         return fail(BGPQ_EHIP, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
     }
-    set_bulk_mem(h);
     int rc = fill_items(h, nullptr);
     if (rc == BGPQ_OK && hipStreamSynchronize(nullptr) != hipSuccess) rc = fail(BGPQ_EHIP, "sync after fill");
     if (rc != BGPQ_OK) {
@@ -440,14 +453,15 @@ static double sort_us(const bgpq_heap* h, long long keys, bool one = false) {
     if (one && bulk_one_tile(h, keys)) return 30.0;
     return 60.0 + keys * (h->key_type == BGPQ_KEY_U64 ? 50e-6 : 15e-6);
 }
+static bool bulk_fits(const bgpq_heap* h, long long keys) { return keys < kBulkMaxKeys && h->bulk.tiles_max > 0; }
 static bool insert_pays(const bgpq_heap* h, long long calls, long long keys) {
-    return keys < kBulkMaxKeys && calls * 2.0 > sort_us(h, keys, true);
+    return bulk_fits(h, keys) && calls * 2.0 > sort_us(h, keys, true);
 }
 static bool delete_pays(const bgpq_heap* h, long long calls, long long keys, bool ascends) {
-    return keys < kBulkMaxKeys && calls * 4.0 > (ascends ? 20.0 + keys * 5e-6 : sort_us(h, keys));
+    return bulk_fits(h, keys) && calls * 4.0 > (ascends ? 20.0 + keys * 5e-6 : sort_us(h, keys));
 }
 static bool sort_pays(const bgpq_heap* h, long long in, long long pops, long long keys) {
-    return keys < kBulkMaxKeys && in * 2.0 + pops * 4.0 > sort_us(h, keys, true);
+    return bulk_fits(h, keys) && in * 2.0 + pops * 4.0 > sort_us(h, keys, true);
 }
 
 // A grid of one workgroup keeps the calls' own order, one after the other;

@@ -2,6 +2,7 @@
 // device memory is host memory, a launch only leaves a note.  It shows what the
 // host decides where no GPU can (a device short of memory) or need (two threads).
 //   capi_host counters   two threads: calls on a heap, and reads of its counters
+//   capi_host memory     heaps that fill the device's memory
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -13,13 +14,20 @@
 using namespace bgpq;
 
 // ------------------------------------------------------------- HIP runtime
+static size_t g_free = ~(size_t)0;  // of the device's memory
+static int g_bulk = 0, g_rows = 0;  // launches
+
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
-    *p = calloc(1, n);
-    return *p ? hipSuccess : hipErrorOutOfMemory;
+    if (n > g_free) return *p = nullptr, hipErrorOutOfMemory;
+    size_t* const q = (size_t*)calloc(1, n + 16);
+    g_free -= *q = n;
+    return *p = q + 2, hipSuccess;
 }
 hipError_t hipFree(void* p) {
-    free(p);
+    size_t* const q = (size_t*)p - 2;
+    g_free += *q;
+    free(q);
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
@@ -55,7 +63,9 @@ hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hi
 
 // ----------------------------------------------------------------- kernels
 namespace bgpq {
-static hipError_t row_insert(const HeapArgs&, const void*, long long, int, int, hipStream_t) { return hipSuccess; }
+static hipError_t row_insert(const HeapArgs&, const void*, long long, int, int, hipStream_t) {
+    return ++g_rows, hipSuccess;
+}
 static hipError_t row_del(const HeapArgs&, void*, long long, int, hipStream_t) { return hipSuccess; }
 static hipError_t row_conc(const HeapArgs&, const void*, long long, int, void*, long long, int, hipStream_t) {
     return hipSuccess;
@@ -83,7 +93,7 @@ hipError_t clear_u32(void*, int*, int*, int, int, uint32_t, hipStream_t) { retur
 hipError_t clear_u64(void*, int*, int*, int, int, uint64_t, hipStream_t) { return hipSuccess; }
 hipError_t bulk_insert(const bgpq_heap*, const void*, long long, void*, long long, long long, int, hipEvent_t, int,
                        hipStream_t) {
-    return hipSuccess;
+    return ++g_bulk, hipSuccess;
 }
 hipError_t bulk_delete(const bgpq_heap*, void*, long long, long long, int, bool, int, hipStream_t) {
     return hipSuccess;
@@ -119,8 +129,32 @@ static int counters() {
     return 0;
 }
 
+static int memory() {
+    const int B = 1024, batches = 1 << 12;
+    const size_t items = sizeof(uint32_t) * B * (batches + 1), status = 128 * (size_t)(batches + 1);
+    uint32_t key = 0;
+    for (const size_t room : {items + status + (64 << 10), items + status - 1, 2 * (items + status)}) {
+        g_free = room;
+        bgpq_heap* h = nullptr;
+        const int rc = bgpq_create(&h, BGPQ_BUITDD, BGPQ_KEY_U32, batches, B, 0xFFFFFFFFu);
+        if (room < items + status) {
+            CHECK(rc == BGPQ_EHIP && !h && g_free == room);
+            continue;
+        }
+        CHECK(rc == BGPQ_OK);
+        g_bulk = g_rows = 0;
+        CHECK(bgpq_insert(h, &key, 1000 * B, 0, 0, nullptr) == BGPQ_OK);
+        // bulk calls only with their memory; the per-batch kernel always follows
+        CHECK(g_rows == 1 && g_bulk == (room > items + status + (64 << 10)));
+        bgpq_destroy(h);
+        CHECK(g_free == room);
+    }
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "counters")) return counters();
+    if (!strcmp(what, "memory")) return memory();
     return 2;
 }

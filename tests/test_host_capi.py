@@ -26,3 +26,10 @@ def test_counters_read_beside_another_threads_calls(built):
     """bgpq_item_count and its like correct the host's count of keys while
     another thread inserts and pops: no data race."""
     _run(built, "capi_host_threads", "counters")
+
+
+def test_heap_that_fills_the_memory(built):
+    """A heap whose slots just fit is made, without the bulk calls' lookback
+    words and without bulk calls; one whose slots do not is refused, and
+    nothing stays allocated."""
+    _run(built, "capi_host", "memory")
