@@ -71,9 +71,14 @@ static HeapArgs args_of(const bgpq_heap* h, long long out_cap = 0) {
     return HeapArgs{h->items, h->status, h->ctr, h->init_limits, h->batch_num, 1, out_cap, nullptr};
 }
 
-// The bulk calls' words follow the counters and, for their lookback, the
-// slots, in the same allocations.  Lookback words are there for the most tiles
-// a bulk sort can have: of keys that take half the slots.
+// The bulk calls' words lie in the same allocations: the plan behind the
+// counters, in their page, the lookback and sort words behind the slots.  (With
+// the sort words behind the counters, the heap's small allocations took eight
+// pages where they took six, the counters came to lie elsewhere, and single
+// calls took up to 1 us longer: 54.2, 53.3, 54.2, 53.3 us an insertion into
+// six heaps made in turn before, 54.5 into each of them then, 64 batches of
+// 2048 u64 keys.)  Lookback words are there for the most tiles a bulk sort can
+// have: of keys that take half the slots.
 static size_t items_bytes(const bgpq_heap* h) {
     return key_bytes(h->key_type) * (size_t)h->batch_size * (size_t)(h->batch_num + 1);
 }
@@ -83,21 +88,20 @@ static int bulk_tiles_max(const bgpq_heap* h) {
     const long long keys = std::min<long long>((long long)(h->batch_num + 1) * h->batch_size / 2, kBulkMaxKeys);
     return (int)(keys / tile + 1);
 }
-static size_t bulk_fixed_bytes() {
-    return up256(ctr_bytes()) + up256(sizeof(BulkPlan)) + up256(sizeof(unsigned) * kSortWords);
-}
+static size_t plan_bytes() { return up256(ctr_bytes()) + sizeof(BulkPlan); }  // counters and plan
 static size_t bulk_look_bytes(const bgpq_heap* h) { return sizeof(unsigned) * kRadix * (size_t)bulk_tiles_max(h); }
-static void set_bulk_mem(bgpq_heap* h, bool look) {
-    char* p = (char*)h->ctr + up256(ctr_bytes());
-    h->bulk.plan = (BulkPlan*)p;
-    p += up256(sizeof(BulkPlan));
-    h->bulk.hist = (unsigned*)p;
-    h->bulk.ticket = h->bulk.hist + kMaxPasses * kRadix;
-    h->bulk.sync = (int*)(h->bulk.ticket + kMaxPasses);
-    p = (char*)h->items + up256(items_bytes(h));
+static size_t bulk_sort_bytes() { return sizeof(unsigned) * kSortWords; }
+static void set_bulk_mem(bgpq_heap* h, bool sorts) {
+    h->bulk = BulkMem{};
+    h->bulk.plan = (BulkPlan*)((char*)h->ctr + up256(ctr_bytes()));
+    if (!sorts) return;
+    char* const p = (char*)h->items + up256(items_bytes(h));
     h->bulk.look[0] = (unsigned*)p;
     h->bulk.look[1] = (unsigned*)(p + bulk_look_bytes(h));
-    h->bulk.tiles_max = look ? bulk_tiles_max(h) : 0;
+    h->bulk.hist = (unsigned*)(p + 2 * bulk_look_bytes(h));
+    h->bulk.ticket = h->bulk.hist + kMaxPasses * kRadix;
+    h->bulk.sync = (int*)(h->bulk.ticket + kMaxPasses);
+    h->bulk.tiles_max = bulk_tiles_max(h);
 }
 
 static int fill_items(bgpq_heap* h, hipStream_t s) {
@@ -106,7 +110,8 @@ static int fill_items(bgpq_heap* h, hipStream_t s) {
                                                : fill_u32(h->items, n, (uint32_t)h->init_limits, s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "fill: %s", hipGetErrorString(e));
     HIPCHK(hipMemsetAsync(h->status, 0, status_bytes(h->batch_num), s));
-    HIPCHK(hipMemsetAsync(h->ctr, 0, bulk_fixed_bytes(), s));  // and the bulk calls' working words
+    HIPCHK(hipMemsetAsync(h->ctr, 0, plan_bytes(), s));
+    if (h->bulk.hist) HIPCHK(hipMemsetAsync(h->bulk.hist, 0, bulk_sort_bytes(), s));
     return BGPQ_OK;
 }
 
@@ -254,16 +259,17 @@ int bgpq_create(bgpq_heap** out, int variant, int key_type, int batch_num, int b
     h->batch_size = batch_size;
     h->init_limits = init_limits;
     h->row = &rows_for(key_type, variant)[bi];
+    h->cus = bgpq_default_grid(batch_size);
     // A device that has no room for the lookback words (up to half a gigabyte)
     // beside the slots: the heap goes without them and without bulk calls.
     size_t bytes = 0;
     hipError_t e = hipSuccess;
     for (const bool bulk : {true, false}) {
         bytes = items_bytes(h);
-        if (bulk) bytes = up256(bytes) + 2 * bulk_look_bytes(h);
+        if (bulk) bytes = up256(bytes) + 2 * bulk_look_bytes(h) + bulk_sort_bytes();
         e = hipMalloc(&h->items, bytes);
         if (e == hipSuccess) e = hipMalloc((void**)&h->status, status_bytes(batch_num));
-        if (e == hipSuccess) e = hipMalloc((void**)&h->ctr, bulk_fixed_bytes());
+        if (e == hipSuccess) e = hipMalloc((void**)&h->ctr, plan_bytes());
         if (e == hipSuccess) {
             set_bulk_mem(h, bulk);
             break;
@@ -439,7 +445,13 @@ static int device_error(bgpq_heap* h) {
     return BGPQ_OK;
 }
 
-static int resolve_grid(bgpq_heap* h, int grid) { return grid > 0 ? grid : bgpq_default_grid(h->batch_size); }
+static int resolve_grid(const bgpq_heap* h, int grid) { return grid > 0 ? grid : h->cus; }
+// Workgroups of a per-batch launch: those beyond the calls would find nothing to
+// do, and starting them took 0.3 to 0.7 us of a pop and an insertion of one
+// batch (72.3 -> 71.6 us, 2048 u64 keys; 101.7 -> 101.0, 4096).
+static int grid_for(const bgpq_heap* h, int grid, long long calls) {
+    return (int)std::min<long long>(resolve_grid(h, grid), calls);
+}
 
 static bool np_variant(const bgpq_heap* h) { return h->variant == BGPQ_BUITDD_NP || h->variant == BGPQ_TDITDD_NP; }
 
@@ -478,7 +490,7 @@ static int insert_calls(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, 
     if (rc) return rc;
     HeapArgs a = args_of(h);
     if (insert_pays(h, (n + chunk - 1) / chunk, h->held + n) && bulk_can(h, d_keys, grid, s)) {
-        const hipError_t e = bulk_insert(h, d_keys, n, nullptr, 0, 0, 0, nullptr, bgpq_default_grid(h->batch_size), s);
+        const hipError_t e = bulk_insert(h, d_keys, n, nullptr, 0, 0, 0, nullptr, h->cus, s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk insert launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
@@ -489,7 +501,7 @@ static int insert_calls(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, 
         a.skip = &h->bulk.plan->go;
     }
     h->held += n;
-    const hipError_t e = h->row->insert(a, d_keys, n, chunk, resolve_grid(h, grid), s);
+    const hipError_t e = h->row->insert(a, d_keys, n, chunk, grid_for(h, grid, (n + chunk - 1) / chunk), s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "insert launch: %s", hipGetErrorString(e));
     return BGPQ_OK;
 }
@@ -503,7 +515,7 @@ static int delete_calls(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t cal
     const long long pops = std::min<long long>(calls, (h->held + h->batch_size - 1) / h->batch_size);
     if (delete_pays(h, pops, h->held, ascends) && bulk_can(h, d_out, grid, s)) {
         const hipError_t e = bulk_delete(h, d_out, out_keys, calls, resolve_grid(h, grid), ascends,
-                                         bgpq_default_grid(h->batch_size), s);
+                                         h->cus, s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk delete launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
@@ -514,7 +526,7 @@ static int delete_calls(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t cal
         a.skip = &h->bulk.plan->go;
     }
     h->held = std::max<long long>(h->held - pops * h->batch_size, 0);
-    const hipError_t e = h->row->del(a, d_out, calls, resolve_grid(h, grid), s);
+    const hipError_t e = h->row->del(a, d_out, calls, grid_for(h, grid, calls), s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "delete launch: %s", hipGetErrorString(e));
     return BGPQ_OK;
 }
@@ -563,7 +575,7 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
     const long long pops = std::min<long long>(calls, (all + h->batch_size - 1) / h->batch_size);
     if (sort_pays(h, in, pops, all) && bulk_can(h, d_keys, grid, s) && bulk_can(h, d_out, grid, s)) {
         const hipError_t e = bulk_insert(h, d_keys, n_insert, d_out, out_keys, calls, grid - grid / 2, nullptr,
-                                         bgpq_default_grid(h->batch_size), s);
+                                         h->cus, s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
         a.skip = &h->bulk.plan->go;
@@ -585,7 +597,7 @@ static int bulk_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n,
     hipEvent_t* const ev = h->sort_events;
     HIPCHK(hipEventRecord(ev[0], s));
     const hipError_t e = bulk_insert(h, d_in, n, d_out, n, pops + 1, poppers, ev[1],
-                                     bgpq_default_grid(h->batch_size), s);
+                                     h->cus, s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk launch: %s", hipGetErrorString(e));
     h->bulk_open = h->ascends = true;
     HIPCHK(hipEventRecord(ev[2], s));

@@ -21,6 +21,7 @@ struct bgpq_heap {
     int* status;
     int* ctr;
     const bgpq::LaunchRow* row;
+    int cus;             // compute units of its device: the default grid
     long long* app_ctl;  // driver control words, allocated on first use
     bgpq::BulkMem bulk;  // working words of the bulk calls, behind ctr and items
     // Keys the heap holds as far as the host can tell without asking the

@@ -3,6 +3,7 @@
 // host decides where no GPU can (a device short of memory) or need (two threads).
 //   capi_host counters   two threads: calls on a heap, and reads of its counters
 //   capi_host memory     heaps that fill the device's memory
+//   capi_host grids      workgroups of the per-batch launches, and what a heap allocates
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -16,6 +17,7 @@ using namespace bgpq;
 // ------------------------------------------------------------- HIP runtime
 static size_t g_free = ~(size_t)0;  // of the device's memory
 static int g_bulk = 0, g_rows = 0;  // launches
+static int g_grid = 0;              // of the last per-batch one
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
@@ -63,12 +65,14 @@ hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hi
 
 // ----------------------------------------------------------------- kernels
 namespace bgpq {
-static hipError_t row_insert(const HeapArgs&, const void*, long long, int, int, hipStream_t) {
-    return ++g_rows, hipSuccess;
+static hipError_t row_insert(const HeapArgs&, const void*, long long, int, int grid, hipStream_t) {
+    return ++g_rows, g_grid = grid, hipSuccess;
 }
-static hipError_t row_del(const HeapArgs&, void*, long long, int, hipStream_t) { return hipSuccess; }
-static hipError_t row_conc(const HeapArgs&, const void*, long long, int, void*, long long, int, hipStream_t) {
-    return hipSuccess;
+static hipError_t row_del(const HeapArgs&, void*, long long, int grid, hipStream_t) {
+    return g_grid = grid, hipSuccess;
+}
+static hipError_t row_conc(const HeapArgs&, const void*, long long, int, void*, long long, int grid, hipStream_t) {
+    return g_grid = grid, hipSuccess;
 }
 static const LaunchRow* rows() {
     static LaunchRow r[kNumBatchSizes];
@@ -152,9 +156,35 @@ static int memory() {
     return 0;
 }
 
+static int grids() {
+    const int B = 64;
+    const size_t before = g_free;
+    bgpq_heap* h = nullptr;
+    CHECK(bgpq_create(&h, BGPQ_BUITDD, BGPQ_KEY_U32, 64, B, 0xFFFFFFFFu) == BGPQ_OK);
+    // the counters' allocation stays in the one page it had without bulk calls
+    CHECK(h->bulk.plan && (char*)(h->bulk.plan + 1) - (char*)h->ctr <= 4096 && g_free < before);
+    uint32_t key = 0;
+    for (int calls : {1, 3, 9})
+        for (int grid : {0, 2, 5, 300}) {
+            const int all = grid ? grid : 256;
+            CHECK(bgpq_insert(h, &key, calls * B - 1, 0, grid, nullptr) == BGPQ_OK);
+            CHECK(g_grid == (all < calls ? all : calls));
+            CHECK(bgpq_delete(h, &key, 1 << 20, calls, grid, nullptr) == BGPQ_OK);
+            CHECK(g_grid == (all < calls ? all : calls));
+            if (grid == 0) continue;
+            // half of a concurrent call's workgroups insert: its grid is what it says
+            CHECK(bgpq_concurrent(h, &key, calls * B, 0, &key, 1 << 20, calls, grid, nullptr) == BGPQ_OK);
+            CHECK(g_grid == grid);
+        }
+    bgpq_destroy(h);
+    CHECK(g_free == before);
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "counters")) return counters();
     if (!strcmp(what, "memory")) return memory();
+    if (!strcmp(what, "grids")) return grids();
     return 2;
 }

@@ -33,3 +33,9 @@ def test_heap_that_fills_the_memory(built):
     words and without bulk calls; one whose slots do not is refused, and
     nothing stays allocated."""
     _run(built, "capi_host", "memory")
+
+
+def test_calls_start_no_idle_workgroups(built):
+    """A call of a few batches starts as many workgroups as it has calls, and
+    the counters share no more memory with the bulk calls' words than a page."""
+    _run(built, "capi_host", "grids")
