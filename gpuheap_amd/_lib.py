@@ -46,6 +46,7 @@ SIGNATURES = {
     "bgpq_default_grid": (c_int, [c_int]),
     "bgpq_test_sort": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p, c_u64, c_int]),
     "bgpq_test_merge": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int]),
+    "bgpq_test_route": (c_int, [c_void_p, c_int_p, c_int_p]),
     "bgpq_gen_keys": (c_int, [c_int, c_u64, c_i64, c_void_p, c_void_p]),
     "bgpq_last_error": (ctypes.c_char_p, []),
     "bgpq_dev_malloc": (c_int, [ctypes.POINTER(c_void_p), c_size_t]),

@@ -153,6 +153,7 @@ int bgpq_on_stream(bgpq_heap* h, hipStream_t s) {
     h->used = true;
     h->stream = s;
     h->ascends = false;
+    h->route = BGPQ_ROUTE_BATCHES;
     return BGPQ_OK;
 }
 
@@ -493,11 +494,13 @@ static int insert_calls(bgpq_heap* h, const void* d_keys, int64_t n, int chunk, 
         const hipError_t e = bulk_insert(h, d_keys, n, nullptr, 0, 0, 0, nullptr, h->cus, s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk insert launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
+        h->route = bulk_one_tile(h, h->held + n) ? BGPQ_ROUTE_TILE : BGPQ_ROUTE_SORT;
         a.skip = &h->bulk.plan->go;
     } else if (n <= chunk && solo_pays(h) && bulk_can(h, d_keys, grid, s)) {
         const hipError_t e = solo_insert(h, d_keys, (int)n, s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "insert launch: %s", hipGetErrorString(e));
         h->bulk_open = true;
+        h->route = BGPQ_ROUTE_SINGLE;
         a.skip = &h->bulk.plan->go;
     }
     h->held += n;
@@ -518,11 +521,13 @@ static int delete_calls(bgpq_heap* h, void* d_out, int64_t out_keys, int64_t cal
                                          h->cus, s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk delete launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
+        h->route = ascends ? BGPQ_ROUTE_COPY : BGPQ_ROUTE_SORT;
         a.skip = &h->bulk.plan->go;
     } else if (calls == 1 && solo_pays(h) && h->held >= h->batch_size && bulk_can(h, d_out, grid, s)) {
         const hipError_t e = solo_delete(h, d_out, out_keys, s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "delete launch: %s", hipGetErrorString(e));
         h->bulk_open = true;
+        h->route = BGPQ_ROUTE_SINGLE;
         a.skip = &h->bulk.plan->go;
     }
     h->held = std::max<long long>(h->held - pops * h->batch_size, 0);
@@ -578,6 +583,7 @@ int bgpq_concurrent(bgpq_heap* h, const void* d_keys, int64_t n_insert, int chun
                                          h->cus, s);
         if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk launch: %s", hipGetErrorString(e));
         h->bulk_open = h->ascends = true;
+        h->route = bulk_one_tile(h, all) ? BGPQ_ROUTE_TILE : BGPQ_ROUTE_SORT;
         a.skip = &h->bulk.plan->go;
     }
     h->held = std::max<long long>(all - pops * h->batch_size, 0);
@@ -600,6 +606,7 @@ static int bulk_heapsort(bgpq_heap* h, const void* d_in, void* d_out, int64_t n,
                                      h->cus, s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "bulk launch: %s", hipGetErrorString(e));
     h->bulk_open = h->ascends = true;
+    h->route = bulk_one_tile(h, n) ? BGPQ_ROUTE_TILE : BGPQ_ROUTE_SORT;
     HIPCHK(hipEventRecord(ev[2], s));
     const hipError_t r = bulk_report(h, h->sort_report, s);
     if (r != hipSuccess) return fail(BGPQ_EHIP, "report launch: %s", hipGetErrorString(r));
@@ -690,6 +697,18 @@ int bgpq_test_merge(int key_type, int batch_size, const void* d_a, const void* d
     hipError_t e = rows[bi].merge(d_a, d_b, d_small, d_large, batches, algo, nullptr);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "merge launch: %s", hipGetErrorString(e));
     HIPCHK(hipDeviceSynchronize());
+    return BGPQ_OK;
+}
+
+int bgpq_test_route(bgpq_heap* h, int* route, int* passes) {
+    if (!h || !route) return fail(BGPQ_EINVAL, "null argument");
+    std::lock_guard<std::recursive_mutex> hold(h->lock);
+    HIPCHK(hipDeviceSynchronize());
+    BulkPlan pl;
+    HIPCHK(hipMemcpy(&pl, h->bulk.plan, sizeof pl, hipMemcpyDeviceToHost));
+    *route = pl.go ? h->route : BGPQ_ROUTE_BATCHES;
+    if (*route == BGPQ_ROUTE_SORT && pl.ascending) *route = BGPQ_ROUTE_COPY;
+    if (passes) *passes = *route == BGPQ_ROUTE_SORT ? pl.active : 0;
     return BGPQ_OK;
 }
 

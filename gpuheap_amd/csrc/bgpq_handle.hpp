@@ -38,6 +38,7 @@ struct bgpq_heap {
     hipEvent_t bulk_done;  // end of the last bulk call, made with the first
     bool bulk_open;        // calls on another stream have to wait for it
     bool ascends;          // like `held`: the last call was a bulk call
+    int route;             // of the last call, if the plan did not refuse (bgpq_route)
     // A heap sort's start, middle and end, and what its end tells the host;
     // made with the first one.
     hipEvent_t sort_events[3];

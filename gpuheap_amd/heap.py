@@ -20,6 +20,7 @@ from ._lib import check, lib
 
 VARIANTS = {"buitdd": 0, "buitdd_np": 1, "tditdd": 2, "tditdd_np": 3}
 KEYS = {"u32": (0, np.uint32), "u64": (1, np.uint64)}
+ROUTES = ("batches", "single", "tile", "sort", "copy")
 CTR_BATCH_COUNT, CTR_PARTIAL, CTR_DELETE_COUNT, CTR_ERROR = 0, 1, 2, 3
 
 
@@ -199,6 +200,14 @@ class Heap:
     def concurrent(self, d_keys, n_insert, d_out, calls, chunk=0, grid=0, out_keys=None):
         check(lib().bgpq_concurrent(self._h, _ptr(d_keys), int(n_insert), int(chunk), _ptr(d_out),
                                     self._cap(d_out, out_keys), int(calls), int(grid), None))
+
+    def route(self):
+        """What did the work of the last of these calls (a test hook): one of
+        ROUTES, and the passes that moved keys where it was a sort of many
+        workgroups (0 otherwise)."""
+        r, n = ctypes.c_int(), ctypes.c_int()
+        check(lib().bgpq_test_route(self._h, ctypes.byref(r), ctypes.byref(n)))
+        return ROUTES[r.value], n.value
 
     def set_cursor(self, value=0):
         check(lib().bgpq_set_cursor(self._h, int(value)))

@@ -157,6 +157,19 @@ int bgpq_test_sort(int key_type, int batch_size, const void* d_in, const int* d_
 int bgpq_test_merge(int key_type, int batch_size, const void* d_a, const void* d_b, void* d_small, void* d_large,
                     int batches, int algo);
 
+/* Test hook: what did the work of the handle's last insertion, deletion,
+ * concurrent call or heap sort (a heap sort of two calls: of the deletion).
+ * *passes, if not null: the sort's passes that moved keys (BGPQ_ROUTE_SORT).
+ * Waits for the device. */
+enum bgpq_route {
+    BGPQ_ROUTE_BATCHES = 0, /* one batch after the other, the heap shared */
+    BGPQ_ROUTE_SINGLE = 1,  /* one batch, one workgroup without locks */
+    BGPQ_ROUTE_TILE = 2,    /* a sort of one workgroup */
+    BGPQ_ROUTE_SORT = 3,    /* a sort of many */
+    BGPQ_ROUTE_COPY = 4     /* pops copied from slots that ascend */
+};
+int bgpq_test_route(bgpq_heap* h, int* route, int* passes);
+
 /* Synthetic heap-sort keys on the device: key i is built from the (i+1)-th
  * SplitMix64 output for `seed`; u32 keys lie in [0, 2^32-2], u64 keys are
  * (u32 key << 32) | i.  Ordered on `stream`. */
