@@ -12,6 +12,7 @@ bounded sample, timed on this host).
 
     python bench.py [--steps K] [--warmup W] [--n LOG2|N] [--variant V] [--batch B]
     python bench.py --sweep            # the heap-sort sweep, one JSON line per config
+    python bench.py --per-batch ...    # either with the kernels that share a heap, a batch at a time
 """
 import argparse
 import ctypes
@@ -35,12 +36,45 @@ HBM_PEAK_GBS = 8000.0
 KEYS = {"u32": (0, np.uint32, 4), "u64": (1, np.uint64, 8)}
 
 
-def alg_bytes(n, s):
-    """HBM bytes of a heap sort of n keys of s bytes, done as one radix sort of
-    s digits (include/bgpq.h, bgpq_heapsort).  Insert phase: the histogram reads
-    the keys and every pass but the last reads and writes them.  Delete phase:
-    the last pass, and the refill of the slots that held them."""
-    return {"insert": n * s * (1 + 2 * (s - 1)), "delete": n * s * 3, "total": n * s * (2 + 2 * s)}
+def levels_sum(m):
+    """S(M) = sum_{k=1..M} floor(log2 k): tree levels below the root summed
+    over the heap sizes 1..M batches."""
+    total, lvl, start = 0, 0, 1
+    while start <= m:
+        end = min(2 * start - 1, m)
+        total += lvl * (end - start + 1)
+        lvl += 1
+        start *= 2
+    return total
+
+
+def alg_bytes(n, b, s, route, passes):
+    """HBM bytes of a heap sort of n keys of s bytes, batch b, by the route it
+    took (Heap.route).
+    sort     insert phase: the histogram reads the keys and each of the passes
+             that move keys, but the last, reads and writes them.  Delete phase:
+             the last pass, and the refill of the free slots that held keys (of
+             the slots in use, too, where the passes are odd).
+    tile     one workgroup reads and writes the keys, in the delete phase.
+    batches  insert reads the input once and reads and writes one batch per
+             level; delete writes the output once, reads two children and writes
+             two nodes per level."""
+    if route == "sort":
+        ins, dele = n * s * (1 + 2 * (passes - 1)), n * s * (3 + passes % 2)
+    elif route == "tile":
+        ins, dele = 0, 2 * n * s
+    else:
+        sm = levels_sum(n // b)
+        ins, dele = n * s + 2 * b * s * sm, n * s + 4 * b * s * sm
+    return {"insert": ins, "delete": dele, "total": ins + dele}
+
+
+def hbm_fracs(n, b, s, r):
+    """Shares of the HBM peak over both phases: of the bytes above, and of the
+    keys read once and written once."""
+    t = (r["ms_insert"] + r["ms_delete"]) / 1e3 * HBM_PEAK_GBS * 1e9
+    return {"hbm_frac_total": alg_bytes(n, b, s, r["route"], r["passes"])["total"] / t,
+            "hbm_frac_keys_once": 2 * n * s / t}
 
 
 def parse_n(v):
@@ -75,13 +109,15 @@ def make_input(n, key, order="random", seed=0):
 
 
 def run_config(n, key, variant, batch, gi, gd, steps, warmup, order="random", seed=0, verify=True, d_in=None,
-               fp_in=None):
+               fp_in=None, per_batch=False):
     kt, dtype, ks = KEYS[key]
     own_in = d_in is None
     if own_in:
         d_in = make_input(n, key, order, seed)
     d_out = DeviceBuffer(n * ks)
     h = Heap(batch_num_for(n, batch), batch, variant=variant, key=key)
+    if per_batch:
+        h.view()  # a heap that others may use at any time
     for _ in range(warmup):
         h.heapsort(d_in, n, grid_insert=gi, grid_delete=gd, d_out=d_out)
     G.sync()
@@ -93,6 +129,7 @@ def run_config(n, key, variant, batch, gi, gd, steps, warmup, order="random", se
         dele.append(b)
     G.sync()
     wall = time.perf_counter() - t0
+    route, passes = h.route()
     ok = None
     if verify:
         if fp_in is None:
@@ -108,7 +145,7 @@ def run_config(n, key, variant, batch, gi, gd, steps, warmup, order="random", se
     d_out.free()
     t_ins, t_del = float(np.mean(ins)), float(np.mean(dele))
     return {"ms_insert": t_ins, "ms_delete": t_del, "ms_step_wall": 1e3 * wall / max(steps, 1),
-            "keys_per_s": n / ((t_ins + t_del) / 1e3), "ok": ok}
+            "keys_per_s": n / ((t_ins + t_del) / 1e3), "route": route, "passes": passes, "ok": ok}
 
 
 def cpu_model():
@@ -444,6 +481,8 @@ def main():
     ap.add_argument("--order", choices=["random", "ascending", "descending"], default="random")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--sweep", action="store_true")
+    ap.add_argument("--per-batch", action="store_true",
+                    help="on a heap whose view was handed out: the lock-coupled kernels instead of the bulk sort")
     ap.add_argument("--sweep-sets", default="u32:random,u32:descending,u64:random",
                     help="key sets of the sweep, key:order pairs")
     ap.add_argument("--calibrate", action="store_true",
@@ -506,10 +545,9 @@ def main():
                     if key == "u64" and b > 4096:
                         continue
                     r = run_config(args.n, key, variant, b, args.grid_insert, args.grid_delete, 1, 0, order=order,
-                                   d_in=d_in, fp_in=fp_in)
-                    ab = alg_bytes(args.n, KEYS[key][2])
+                                   d_in=d_in, fp_in=fp_in, per_batch=args.per_batch)
                     r.update({"n": args.n, "key": key, "order": order, "variant": variant, "batch": b,
-                              "hbm_frac_total": ab["total"] / ((r["ms_insert"] + r["ms_delete"]) / 1e3) / 8e12})
+                              **hbm_fracs(args.n, b, KEYS[key][2], r)})
                     print(json.dumps(r), flush=True)
             d_in.free()
         return
@@ -524,20 +562,23 @@ def main():
     d_in = make_input(args.n, args.key, args.order)
     fp_in = fingerprint(d_in.to_numpy(KEYS[args.key][1], args.n))
     r = run_config(args.n, args.key, args.variant, args.batch, args.grid_insert, args.grid_delete, args.steps,
-                   args.warmup, order=args.order, d_in=d_in, fp_in=fp_in)
+                   args.warmup, order=args.order, d_in=d_in, fp_in=fp_in, per_batch=args.per_batch)
     if not r["ok"]:
         print("[bench] output check FAILED", file=sys.stderr, flush=True)
     s = KEYS[args.key][2]
-    ab = alg_bytes(args.n, s)
+    ab = alg_bytes(args.n, args.batch, s, r["route"], r["passes"])
     dom = "delete" if r["ms_delete"] >= r["ms_insert"] else "insert"
-    dom_ms = r["ms_" + dom]
-    achieved = ab[dom] / (dom_ms / 1e3) / 1e9
+    achieved = ab[dom] / (r["ms_" + dom] / 1e3) / 1e9
     workload = f"heapsort_{args.key}_n{args.n}_{args.variant}_b{args.batch}_{args.order}"
-    measured = traffic_for(workload)
-    kernel = f"k_bulk_hist + {s - 1} k_bulk_pass" if dom == "insert" else "k_bulk_pass + k_bulk_finish"
+    measured = traffic_for(workload) or {}
+    if r["route"] == "sort":
+        kernel = f"k_bulk_hist + {r['passes'] - 1} k_bulk_pass" if dom == "insert" else "k_bulk_pass + k_bulk_finish"
+        traffic = measured.get(dom)
+    else:
+        kernel = "k_bulk_tile" if r["route"] == "tile" else f"k_{dom}"
+        traffic = measured.get(kernel)
     roofline = {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS,
-                "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-                "traffic": measured.get(dom) if measured else None,
+                "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                 "alg_bytes_per_launch": ab[dom]}
     ok = bool(r["ok"])
     line = {
@@ -557,7 +598,8 @@ def main():
                    "n_keys": args.n, "key": args.key, "variant": args.variant, "batch_size": args.batch,
                    "grid_insert": args.grid_insert, "grid_delete": args.grid_delete, "order": args.order},
         "phases_ms": {"insert": r["ms_insert"], "delete": r["ms_delete"]},
-        "hbm_frac_total": ab["total"] / ((r["ms_insert"] + r["ms_delete"]) / 1e3) / (HBM_PEAK_GBS * 1e9),
+        "route": r["route"],
+        **hbm_fracs(args.n, args.batch, s, r),
         "check": "output sorted and multiset fingerprint equal to input: " + ("ok" if r["ok"] else "FAILED"),
         "roofline": roofline,
     }
@@ -568,12 +610,10 @@ def main():
             continue
         print(f"[bench] heap sort at B={b}", file=sys.stderr, flush=True)
         e = run_config(args.n, args.key, args.variant, b, args.grid_insert, args.grid_delete, 1, 1,
-                       order=args.order, d_in=d_in, fp_in=fp_in)
+                       order=args.order, d_in=d_in, fp_in=fp_in, per_batch=args.per_batch)
         ok = ok and bool(e["ok"])
-        ab_b = alg_bytes(args.n, s)
         extras[str(b)] = {"keys_per_s": e["keys_per_s"], "ms_insert": e["ms_insert"], "ms_delete": e["ms_delete"],
-                          "hbm_frac_total": ab_b["total"] / ((e["ms_insert"] + e["ms_delete"]) / 1e3) /
-                          (HBM_PEAK_GBS * 1e9), "check": "ok" if e["ok"] else "FAILED"}
+                          **hbm_fracs(args.n, b, s, e), "check": "ok" if e["ok"] else "FAILED"}
     if extras:
         line["other_batch_sizes"] = extras
     d_in.free()
