@@ -61,7 +61,7 @@ struct BulkPlan {
     // termination vote: deletions that found nothing, and workgroups left busy
     int idle, busy;
     int active;           // passes that move keys: the last launches
-    int digit[kMaxPasses];  // the digit of each of them
+    int order[kMaxPasses];  // of a launch: its pass's position << 8 | its digit, -1: none
     int through_out;        // the passes alternate between the free slots and the output
 };
 
