@@ -339,8 +339,8 @@ __device__ __forceinline__ unsigned rank_of(const unsigned (&rank)[H], int u) {
     return u % 2 == 0 ? rank[u / 2] & 0xFFFFu : rank[u / 2] >> 16;
 }
 // Ranks of the wave's keys, U rows of 64, among those of the same digit, in
-// order, and the digits' counts in `mine` (zeroed before).  About 80 vector
-// instructions and 3 LDS accesses a row.  A lane finds the lanes with its
+// order, and the digits' counts in `mine` (zeroed before): most of a pass's
+// vector instructions, and 3 LDS accesses a row.  A lane finds the lanes with its
 // digit bit by bit: one ballot and one v_bitop3 for each half of the mask.
 // The ranks are kept two to a register: with 32 rows' keys and ranks in
 // registers of their own the large tiles of u32 keys spilled, which wrote 1.7
@@ -410,8 +410,8 @@ __device__ __forceinline__ void count_digits(const unsigned (&cnt)[W][kRadix], u
 //   * 256 threads, one per digit, publish the tile's counts and look back
 //     for those of the tiles before it; meanwhile the keys move into LDS in
 //     digit order, from where each digit's run is written as a whole.
-// What bounds it: vector instructions (75 for 64 keys, 70% of the time at 2^28
-// u32 keys) and waits for LDS and memory; 700 us a pass there, 3.1 TB/s read
+// What bounds it: vector instructions (69 for 64 keys, 75% of the cycles at 2^28
+// u32 keys) and waits for LDS and memory; 694 us a pass there, 3.1 TB/s read
 // and written where a copy reaches 4.6.  It took 1150 us with lane masks built
 // by selects (95 instructions for the ranks alone; a mask's step is one
 // v_bitop3 now) and a look-back of one tile at a time, each a round trip of

@@ -7,7 +7,17 @@
 // needs neither the locks nor the waits for its stores, and the batches of the
 // levels to come are loaded while the present one is merged: an insertion's
 // path is known from its slot, a pop's next level once its children have been
-// compared.  SOLO_FIGURES
+// compared.
+//
+// One insertion and one pop, 1024 batches held, the host's part and the wait
+// included (us; shared kernels, here):
+//   u32  B = 64    37 and 39, 23 and 26      u64  B = 64   39 and 41, 26 and 28
+//        256       40 and 43, 25 and 28           256      46 and 51, 31 and 34
+//        1024      45 and 44, 32 and 36           512      53 and 56, 38 and 42
+//        4096      57 and 56, 46 and 47           1024     59 and 53, 57 and 62
+// u64 keys from B = 1024 on, where the shared sift takes its merges by halves,
+// and u32 keys of B = 8192 stay with the shared kernels (solo_pays; beyond that
+// line B = 2048 u64 has 67 and 64, 62 and 61, and 8192 u32 77 and 75, 72 and 67).
 //
 // The heap that is left is one that any order of calls could have left: the
 // same counters, every status word AVAIL, free slots at init_limits.  A call

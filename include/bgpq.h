@@ -43,7 +43,11 @@ typedef struct bgpq_heap bgpq_heap;
  * (the delete workspace, 3*batch_size*sizeof(key), must fit gfx950's 160 KB of LDS).
  * Every slot is filled with init_limits on the device; keys inserted later
  * must be strictly below init_limits.  The heap-sort output cursor
- * (deleteCount, the reference's -DHEAP_SORT mode) is always maintained. */
+ * (deleteCount, the reference's -DHEAP_SORT mode) is always maintained.
+ * Calls with many batches are done as one sort where the free slots hold as
+ * many keys again (batch_num at least twice the batches held and inserted, the
+ * reference harness's sizing), the calls come on one stream, none captured, and
+ * the view was not handed out; otherwise a batch at a time, many times slower. */
 int bgpq_create(bgpq_heap** out, int variant, int key_type, int batch_num, int batch_size,
                 uint64_t init_limits);
 /* ~Heap() -- heap/buitdd/heap.cuh:94-116 */
