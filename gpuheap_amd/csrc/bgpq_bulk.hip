@@ -655,6 +655,14 @@ __global__ void k_bulk_report(const BulkPlan* pl, const int* ctr, int* report) {
 }
 static_assert(CTR_WORDS < kReportWords, "report words");
 
+__global__ __launch_bounds__(256) void k_zero_words(int* status, long long nstatus, int* ctr, int nctr,
+                                                    unsigned* sort, int nsort) {
+    const long long i0 = blockIdx.x * 256ll + threadIdx.x, step = gridDim.x * 256ll;
+    for (long long i = i0; i < nstatus; i += step) status[i] = 0;
+    for (long long i = i0; i < nctr; i += step) ctr[i] = 0;
+    for (long long i = i0; i < nsort; i += step) sort[i] = 0;
+}
+
 inline int blocks_for(long long items, int per_block, int most) {
     const long long b = (items + per_block - 1) / per_block;
     return (int)(b < 1 ? 1 : (b > most ? most : b));
@@ -756,6 +764,12 @@ hipError_t bulk_insert(const bgpq_heap* h, const void* keys, long long n, void* 
 }
 bool bulk_one_tile(const bgpq_heap* h, long long keys) {
     return keys <= (h->key_type == BGPQ_KEY_U64 ? bulk_tile<uint64_t>() : bulk_tile<uint32_t>());
+}
+hipError_t zero_words(int* status, long long nstatus, int* ctr, int nctr, unsigned* sort, int nsort, hipStream_t s) {
+    (void)hipGetLastError();  // report this launch only
+    hipLaunchKernelGGL(k_zero_words, dim3(blocks_for(nstatus, 1024, 2048)), dim3(256), 0, s, status, nstatus, ctr, nctr,
+                       sort, nsort);
+    return hipGetLastError();
 }
 hipError_t bulk_report(const bgpq_heap* h, int* report, hipStream_t s) {
     hipLaunchKernelGGL(k_bulk_report, dim3(1), dim3(64), 0, s, h->bulk.plan, h->ctr, report);

@@ -88,6 +88,7 @@ static int bulk_tiles_max(const bgpq_heap* h) {
     const long long keys = std::min<long long>((long long)(h->batch_num + 1) * h->batch_size / 2, kBulkMaxKeys);
     return (int)(keys / tile + 1);
 }
+static_assert(sizeof(BulkPlan) % 4 == 0, "cleared in words");
 static size_t plan_bytes() { return up256(ctr_bytes()) + sizeof(BulkPlan); }  // counters and plan
 static size_t bulk_look_bytes(const bgpq_heap* h) { return sizeof(unsigned) * kRadix * (size_t)bulk_tiles_max(h); }
 static size_t bulk_sort_bytes() { return sizeof(unsigned) * kSortWords; }
@@ -108,10 +109,12 @@ static int fill_items(bgpq_heap* h, hipStream_t s) {
     const long long n = (long long)(h->batch_num + 1) * h->batch_size;
     hipError_t e = h->key_type == BGPQ_KEY_U64 ? fill_u64(h->items, n, h->init_limits, s)
                                                : fill_u32(h->items, n, (uint32_t)h->init_limits, s);
+    // a kernel for the words, too: a caller may capture a reset, and memset
+    // nodes of a graph have given wrong results on later replays
+    if (e == hipSuccess)
+        e = zero_words(h->status, (long long)(status_bytes(h->batch_num) / 4), h->ctr, (int)(plan_bytes() / 4),
+                       h->bulk.hist, h->bulk.hist ? kSortWords : 0, s);
     if (e != hipSuccess) return fail(BGPQ_EHIP, "fill: %s", hipGetErrorString(e));
-    HIPCHK(hipMemsetAsync(h->status, 0, status_bytes(h->batch_num), s));
-    HIPCHK(hipMemsetAsync(h->ctr, 0, plan_bytes(), s));
-    if (h->bulk.hist) HIPCHK(hipMemsetAsync(h->bulk.hist, 0, bulk_sort_bytes(), s));
     return BGPQ_OK;
 }
 

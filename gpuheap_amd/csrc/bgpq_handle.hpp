@@ -71,6 +71,8 @@ bool bulk_one_tile(const bgpq_heap* h, long long keys);
 hipError_t bulk_report(const bgpq_heap* h, int* report, hipStream_t s);
 hipError_t bulk_delete(const bgpq_heap* h, void* out, long long out_cap, long long calls, int poppers, bool ascends,
                        int cus, hipStream_t s);
+// A heap's status words, counters and plan, and sort words to 0.
+hipError_t zero_words(int* status, long long nstatus, int* ctr, int nctr, unsigned* sort, int nsort, hipStream_t s);
 // bgpq_solo.hip: one insertion of `size` keys, one pop; like bulk calls, with
 // plan->go.  solo_pays: the batch sizes where they are the faster ones.
 bool solo_pays(const bgpq_heap* h);

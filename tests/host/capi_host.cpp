@@ -102,6 +102,12 @@ hipError_t bulk_insert(const bgpq_heap*, const void*, long long, void*, long lon
 hipError_t bulk_delete(const bgpq_heap*, void*, long long, long long, int, bool, int, hipStream_t) {
     return hipSuccess;
 }
+hipError_t zero_words(int* status, long long nstatus, int* ctr, int nctr, unsigned* sort, int nsort, hipStream_t) {
+    memset(status, 0, 4 * nstatus);
+    memset(ctr, 0, 4 * nctr);
+    if (nsort) memset(sort, 0, 4 * nsort);
+    return hipSuccess;
+}
 hipError_t bulk_report(const bgpq_heap*, int*, hipStream_t) { return hipSuccess; }
 bool bulk_one_tile(const bgpq_heap*, long long) { return false; }
 bool solo_pays(const bgpq_heap*) { return true; }

@@ -448,3 +448,41 @@ def test_delete_phase_hands_the_keys_out(gpu, key, n, bits):
     print(f"[case] delete phase {ms[0]:.3f} ms, {bits}-bit keys {ms[1]:.3f} ms", flush=True)
     assert ms[1] > 0.5 * ms[0]
     h.close()
+
+
+@pytest.mark.parametrize("key", ["u32", "u64"])
+def test_captured_reset(gpu, key):
+    """A captured reset, insertion and pop: every replay starts from an empty
+    heap, whatever eager calls did between."""
+    print(f"[case] captured reset {key}", flush=True)
+    hip = ctypes.CDLL("libamdhip64.so")
+    s, graph, run = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+    B, n = 128, 128 * 20
+    keys = _keys(key, n, 16, "random")
+    d, out = DeviceBuffer.from_numpy(keys), DeviceBuffer(keys.nbytes)
+    h = Heap(64, B, key=key)
+    h.view()
+    h.insert(d, n)  # loads what a first launch loads
+    h.delete(out, 2)
+    h.reset()
+    G.sync()
+    assert hip.hipStreamBeginCapture(s, 0) == 0
+    check(lib().bgpq_reset(h._h, s))
+    check(lib().bgpq_insert(h._h, d.ptr, n, 0, 0, s))
+    check(lib().bgpq_delete(h._h, out.ptr, n, 3, 1, s))
+    assert hip.hipStreamEndCapture(s, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    want = np.sort(keys)
+    for i in range(4):
+        assert hip.hipGraphLaunch(run, s) == 0
+        assert hip.hipStreamSynchronize(s) == 0
+        _valid(h, want[3 * B:])
+        assert h.snapshot()[2][2] == 3 * B
+        assert np.array_equal(out.to_numpy(keys.dtype, 3 * B), want[:3 * B])
+        h.insert(d, 5 * B - 7)  # eager
+        h.delete(out, i)
+        G.sync()
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    h.close()
+    assert hip.hipStreamDestroy(s) == 0
