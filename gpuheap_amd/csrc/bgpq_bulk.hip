@@ -42,11 +42,16 @@ __device__ __forceinline__ int digit_of(K k, int pass) {
     return (int)((k >> (8 * pass)) & (K)(kRadix - 1));
 }
 
-// The loop behind it starts on a line of the instruction cache.  A pass's loops
-// are long and run from there again and again: where they happened to start
-// made up to 2% of a sort (12.3 M descending u32 keys 276.5 and 283 us with the
-// same instructions 16 bytes apart, 279 aligned; 2^28 random 3197, 3207, 3174).
-#define BULK_ALIGN_LOOP() asm volatile(".p2align 6")
+// The loop behind it starts on a line of the instruction cache, in a pass of the
+// large tiles.  Its loops are long and run from there again and again: where
+// they happened to start made up to 2% of a sort (12.3 M descending u32 keys 276.5
+// and 283 us with the same instructions 16 bytes apart, 279 aligned; 2^28 random
+// 3197, 3207, 3174).  In a pass of the small tiles it gained nothing (rounds of
+// 1.5 M u64 keys in all 971 us, 967 without).
+template <typename K, int T>
+__device__ __forceinline__ void align_loop() {
+    if constexpr (T == bulk_tile<K>(true)) asm volatile(".p2align 6");
+}
 
 // The same value as one the compiler knows nothing of: what is computed from
 // it is computed anew, not kept in registers from the last use on.
@@ -442,7 +447,7 @@ __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, in
     unsigned* const look = a.mem.look[ord & 1];
     unsigned* const next = last ? nullptr : a.mem.look[(ord & 1) ^ 1];
     const unsigned start = t < kRadix ? a.mem.hist[pass * kRadix + t] : 0;
-    BULK_ALIGN_LOOP();
+    align_loop<K, T>();
     for (;;) {
         if (t == 0) s_tile = (int)atomicAdd(a.mem.ticket + pass, 1u);
 #pragma unroll
@@ -495,7 +500,7 @@ __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, in
         if (t < kRadix && tile > 0) {
             const unsigned* const p = look + t;
             int back = tile - 1, polls = 0;
-            BULK_ALIGN_LOOP();
+            align_loop<K, T>();
             for (bool open = true; open;) {
                 unsigned v[kWindow];
 #pragma unroll
@@ -526,7 +531,7 @@ __global__ __launch_bounds__(kBulkThreads, 4) void k_bulk_pass(BulkArgs<K> a, in
         if (here == T && !split) {
             // eight at a time: all of them would take more registers than
             // the workgroups on a CU leave each other
-            BULK_ALIGN_LOOP();
+            align_loop<K, T>();
 #pragma unroll 1
             for (int u = 0; u < U; u += 8) {
 #pragma unroll
